@@ -69,6 +69,16 @@ int kq_gemv_multi(int n, const void* const* w, const int* R, int C, const int* t
                   const float* x, float* const* y, void* stream);
 
 /*
+ * The same for N rows of x (row stride ldx floats, any N >= 1): y[i] holds N rows (row stride ldy[i]
+ * floats, at least R[i]), each equal to kq_gemv_multi on that row bit for bit.  The fp32 form of the
+ * batched layout y[ntok][R] (tc.cu:306-310): prompts and drafted tokens in the reference's own
+ * numerics, which the reference's Q4 engine feeds token by token (gpu4.py:109-110), with the weights
+ * read and unpacked once per 8 rows instead of once per row.  One launch per weight type.
+ */
+int kq_gemv_rows(int n, const void* const* w, const int* R, int C, const int* type, const float* x, int64_t ldx,
+                 int N, float* const* y, const int64_t* ldy, void* stream);
+
+/*
  * Q8_K activation quantizer (GGML quantize_row_q8_K_ref semantics; no counterpart in the
  * reference, whose Q4 path keeps activations in fp32, q4kernels.h:37-83).  x: N rows of C floats
  * with row stride ldx (floats), 4-byte aligned; xq: N*(C/256) blocks of 292 B, 4-byte aligned.

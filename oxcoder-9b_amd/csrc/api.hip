@@ -118,6 +118,39 @@ int kq_gemv_multi(int n, const void* const* w, const int* R, int C, const int* t
     return check_launch(fn);
 }
 
+int kq_gemv_rows(int n, const void* const* w, const int* R, int C, const int* type, const float* x, int64_t ldx,
+                 int N, float* const* y, const int64_t* ldy, void* stream) {
+    static const char* fn = "kq_gemv_rows";
+    if (n < 1 || n > 3) return fail(KQ_ERR_ARG, "%s: n=%d must be 1..3", fn, n);
+    if (!w || !R || !type || !y || !ldy) return fail(KQ_ERR_ARG, "%s: NULL array argument", fn);
+    if (N < 1) return fail(KQ_ERR_ARG, "%s: N=%d must be positive", fn, N);
+    if (N == 1) return kq_gemv_multi(n, w, R, C, type, x, y, stream);
+    int64_t tiles = 0;
+    for (int i = 0; i < n; i++) {
+        KQ_TRY(check_matrix(w[i], R[i], C, type[i], fn));
+        KQ_TRY(check_ptr(y[i], 4, "y[i]", fn));
+        if (ldy[i] < R[i]) return fail(KQ_ERR_ARG, "%s: ldy[%d] is smaller than R", fn, i);
+        tiles += R[i] / 8;
+    }
+    if (tiles > (1 << 27)) return fail(KQ_ERR_ARG, "%s: too many rows in one call", fn);
+    if (ldx < 0) return fail(KQ_ERR_ARG, "%s: ldx=%lld is negative", fn, (long long)ldx);
+    KQ_TRY(check_ptr(x, 4, "x", fn));
+    for (int ty : {KQ_TYPE_Q4_K, KQ_TYPE_Q6_K}) {
+        const uint8_t* ws[3];
+        int rs[3];
+        float* ys[3];
+        int64_t ls[3];
+        int k = 0;
+        for (int i = 0; i < n; i++)
+            if (type[i] == ty) {
+                ws[k] = static_cast<const uint8_t*>(w[i]); rs[k] = R[i]; ys[k] = y[i]; ls[k] = ldy[i];
+                k++;
+            }
+        if (k) launch_gemv_f32_rows(k, ws, rs, C, ty, x, ldx, N, ys, ls, as_stream(stream));
+    }
+    return check_launch(fn);
+}
+
 int kq_q8k_quantize(const float* x, int64_t ldx, int C, int N, void* xq, void* stream) {
     static const char* fn = "kq_q8k_quantize";
     if (C <= 0 || C % 256) return fail(KQ_ERR_ARG, "%s: C=%d must be a positive multiple of 256", fn, C);

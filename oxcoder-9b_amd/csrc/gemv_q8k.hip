@@ -161,10 +161,10 @@ __device__ __forceinline__ void load_frag(Frag<TYPE_Q4_K>& f, const uint8_t* bk,
 // the scale window [192 + 8h, 200 + 8h) and d [208, 210) are read from the dword-aligned address
 // at or below them; for even rows (block start = 0 mod 4) the last word read reaches 2 bytes
 // into the next row's block, which exists because row 7 of a tile is odd.
-__device__ __forceinline__ void load_frag(Frag<TYPE_Q6_K>& f, const uint8_t* bk, int p) {
+__device__ __forceinline__ void load_frag(Frag<TYPE_Q6_K>& f, const uint8_t* bk, int p, uint32_t sh) {
     const int h = p >> 1, jj = p & 1;
     // pointer arithmetic (not an integer round trip) keeps the global address space
-    f.sh = uint32_t(reinterpret_cast<uintptr_t>(bk) & 3);   // the same shift for every field
+    f.sh = sh;                                      // the same shift for every field
     const uint8_t* b4 = bk - f.sh;
     f.l0 = ld16_a4(b4 + h * 64 + 16 * jj);          // ql bytes 64h + 16jj ..
     f.l1 = ld16_a4(b4 + h * 64 + 32 + 16 * jj);     // ql bytes 64h + 32 + 16jj ..
@@ -172,6 +172,14 @@ __device__ __forceinline__ void load_frag(Frag<TYPE_Q6_K>& f, const uint8_t* bk,
     f.sc4 = ld16_a4(b4 + 192);                      // the 16 scales
     f.dw = ld4(b4 + 208);                           // d
 }
+__device__ __forceinline__ void load_frag(Frag<TYPE_Q6_K>& f, const uint8_t* bk, int p) {
+    load_frag(f, bk, p, uint32_t(reinterpret_cast<uintptr_t>(bk) & 3));
+}
+// The same for row r of a tile column, r known when compiling: blocks of odd rows start at 2 (mod 4).
+__device__ __forceinline__ void load_frag_row(Frag<TYPE_Q6_K>& f, const uint8_t* bk, int p, int r) {
+    load_frag(f, bk, p, 2u * (uint32_t)(r & 1));
+}
+__device__ __forceinline__ void load_frag_row(Frag<TYPE_Q4_K>& f, const uint8_t* bk, int p, int) { load_frag(f, bk, p); }
 // The fields a lane multiplies.  Quad lane p = 2h + jj holds the 16-B chunks at block offsets
 // (relative to the dword-aligned start) l0: 64h + 16jj, l1: 64h + 32 + 16jj, hb: 128 + 32h + 16jj,
 // so the dword following
@@ -889,6 +897,259 @@ k_gemv_q8k_split2(KQ_GEMV_HEAD, int nwgA, MatGroup mgA, MatGroup mgB, uint8_t* x
                                                   nullptr, X, xs, nullptr);
 }
 
+// ------------------------------------------------------------------ several rows of fp32 activations
+// N rows of fp32 activations against the same weights (drafted tokens and prompts in the reference's
+// numerics), every output with the bits of the one-row kernel: the same lanes, the same fp32 chain per
+// sub-block and the same trees, so only the loops around them differ.  One row at a time reads and
+// unpacks every weight once per row; here a workgroup holds one column pass (4096 columns) of up to T
+// rows in LDS, and each wave unpacks a unit of FR_ROWS weight rows once, into f16 operands in registers,
+// and multiplies it with each of the T rows.  The multiply-adds are then the bound, one per weight and
+// row: 256 of the ~350 VALU instructions a wave spends per unit and row of x.  The lanes' sums of four
+// weight rows go through one slot tree (fr_slot_tree).  Each activation read from LDS serves FR_ROWS
+// rows.  Measured, one-row launches -> this kernel, us: 24576x4096 Q4_K at N = 2 / 5 28.9 / 69.8 -> 18.7
+// / 30.9, at N = 24 113 (61 for the multiply-adds alone at 2.4 GHz); 4096x12288 Q6_K at N = 2 / 5 25.2 /
+// 60.3 -> 22.6 / 31.1; 1024x4096 Q4_K at N = 2 8.9 -> 4.9: faster at every size from two rows on.  A
+// 24-row prompt through the 9B layer 1330 -> 260.
+constexpr int FR_ROWS = 4;                  // weight rows per unit
+#ifndef KQ_FR_AHEAD
+#define KQ_FR_AHEAD 3
+#endif
+constexpr int FR_AHEAD = KQ_FR_AHEAD;       // activation chunks read ahead of their use
+template <int T> constexpr int FR_PART = 512 * T;   // floats of pass values a workgroup holds (several column passes)
+
+// One weight row's quarter of a super-block, unpacked: c[] holds the codes as f16 halves in the order
+// dot_halves_f32 takes them (two dwords per four activations), s[] the factors of the epilogue.
+struct FrRow { uint32_t c[32]; float s[4]; };
+__device__ __forceinline__ void fr_unpack(FrRow& o, const Frag<TYPE_Q4_K>& f, int p) {
+    const ScMin sm = q4k_scmin_pair(f.hdr.y, f.hdr.z, f.hdr.w, p);
+    const uint32_t q[8] = {f.qa.x, f.qa.y, f.qa.z, f.qa.w, f.qb.x, f.qb.y, f.qb.z, f.qb.w};
+#pragma unroll
+    for (int k = 0; k < 8; k++) {           // chunk k: elements 4k .. 4k+3 (low nibbles), chunk 8 + k: high nibbles
+        const uint32_t odd = odd_bytes(q[k]);
+        o.c[2 * k] = q[k] & 0x000f000fu;
+        o.c[2 * k + 1] = odd & 0x000f000fu;
+        o.c[16 + 2 * k] = q[k] & 0x00f000f0u;
+        o.c[17 + 2 * k] = odd & 0x00f000f0u;
+    }
+    const float d = f16_lo(f.hdr.x), dm = f16_hi(f.hdr.x);
+    o.s[0] = __fmul_rn(d, (float)sm.sc_lo);
+    o.s[1] = __fmul_rn(d, (float)sm.sc_hi);
+    o.s[2] = __fmul_rn(dm, (float)sm.m_lo);
+    o.s[3] = __fmul_rn(dm, (float)sm.m_hi);
+}
+__device__ __forceinline__ void fr_unpack(FrRow& o, const Q6Fields& f, int p) {
+    const int jj = p & 1;
+    const uint32_t w0 = __builtin_amdgcn_alignbyte(f.sc.y, f.sc.x, f.sh);   // scales 8h .. 8h+3
+    const uint32_t w1 = __builtin_amdgcn_alignbyte(f.sce, f.sc.y, f.sh);    // scales 8h+4 .. 8h+7
+    const u32x4 l0 = funnel(f.l0, f.l0e, f.sh), l1 = funnel(f.l1, f.l1e, f.sh), hb = funnel(f.hb, f.hbe, f.sh);
+    const uint32_t L0[4] = {l0.x, l0.y, l0.z, l0.w}, L1[4] = {l1.x, l1.y, l1.z, l1.w};
+    const uint32_t H[4] = {hb.x, hb.y, hb.z, hb.w};
+#pragma unroll
+    for (int w = 0; w < 4; w++) {           // chunk 4k + w: elements 4w .. 4w+3 of group k
+        const uint32_t m4 = 0x0f0f0f0fu, m2 = 0x30303030u;
+        const uint32_t c[4] = {(L0[w] & m4) | ((H[w] << 4) & m2), (L1[w] & m4) | ((H[w] << 2) & m2),
+                               ((L0[w] >> 4) & m4) | (H[w] & m2), ((L1[w] >> 4) & m4) | ((H[w] >> 2) & m2)};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            o.c[2 * (4 * k + w)] = even_bytes(c[k]);
+            o.c[2 * (4 * k + w) + 1] = odd_bytes(c[k]);
+        }
+    }
+    const float d = f16_lo(f.dw >> (8 * f.sh));
+    const int sc[4] = {sbyte(w0, jj), sbyte(w0, jj + 2), sbyte(w1, jj), sbyte(w1, jj + 2)};
+#pragma unroll
+    for (int k = 0; k < 4; k++) o.s[k] = __fmul_rn(d, (float)sc[k]);
+}
+
+// A lane's 64 activations of a super-block as 16 chunks of 4: the first element of chunk c of part p.
+template <int TYPE> __device__ __forceinline__ int fr_elem(int p, int c) {
+    return TYPE == TYPE_Q4_K ? 64 * p + 4 * c : 128 * (p >> 1) + 32 * (c >> 2) + 16 * (p & 1) + 4 * (c & 3);
+}
+// Accumulator chains per row: the two sub-blocks of a Q4_K quarter, the four of a Q6_K one.
+template <int TYPE> constexpr int FR_NACC = TYPE == TYPE_Q4_K ? 2 : 4;
+
+// slot_tree_f32 for a value per lane of each quad (four trees at once): the same pairs in the same
+// order, by row shifts (lane j <- lane j + 4, then j + 8) instead of the mirrors, which would swap the
+// quad's lanes.  Valid in lanes 0..3.
+__device__ __forceinline__ float fr_slot_tree(float v) {
+    v = __fadd_rn(v, dppf<0x104>(v));      // row_shl:4: quads (0, 1) and (2, 3)
+    v = __fadd_rn(v, dppf<0x108>(v));      // row_shl:8
+    v = xor16_sum(v);
+    return xor32_sum(v);
+}
+
+struct FrArgs {
+    const float* x;
+    int64_t ldx;
+    int N, G, total_units, upw, ntg, tpg, nrb;   // upw: units per workgroup, tpg: rows of x per token group
+    MatGroup mg;                                 // first_unit in units of FR_ROWS rows
+};
+
+template <int TYPE, int T, int W, bool ONEPASS>
+__global__ void __launch_bounds__(64 * W, 2)
+k_gemv_f32_rows(FrArgs a) {
+    constexpr int BS = TYPE == TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES;
+    constexpr int WPT = 8 / FR_ROWS;
+    constexpr int NACC = FR_NACC<TYPE>;
+    // [token][chunk][lane]: a wave's read of one chunk is one contiguous 1 KB
+    __shared__ f32x4 act[T][16][64];
+    __shared__ float sums[T][64][NACC];          // Q4_K: sums of the two sub-blocks; Q6_K: 32 * sum of each
+    __shared__ float part[ONEPASS ? 1 : FR_PART<T>];            // [unit][row][token][pass] when there are several passes
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p = lane & 3, slot = lane >> 2;
+    // the token groups of one block of rows are consecutive workgroups of one die: its L2 serves the
+    // weights to all but the first
+    const int j = blockIdx.x / KQ_XCDS;
+    const int tg = j % a.ntg, rb = (j / a.ntg) * KQ_XCDS + blockIdx.x % KQ_XCDS;
+    if (rb >= a.nrb) return;
+    const int u0 = rb * a.upw, u1 = u0 + a.upw < a.total_units ? u0 + a.upw : a.total_units;
+    const int n0 = tg * a.tpg, nt = a.N - n0 < a.tpg ? a.N - n0 : a.tpg;
+    const int G = a.G, P = ONEPASS ? 1 : (G + 15) >> 4;
+
+    auto unit = [&](int u, int& m, int64_t& row0) -> const uint8_t* {
+        m = u >= a.mg.first_unit[1] ? (u >= a.mg.first_unit[2] ? 2 : 1) : 0;
+        const int v = u - a.mg.first_unit[m];
+        row0 = (int64_t)v * FR_ROWS;
+        return a.mg.w[m] + (int64_t)(v / WPT) * G * (8 * BS) + (v % WPT) * FR_ROWS * BS;
+    };
+    // bit selects (conditional expressions became branches)
+    const uint32_t p1 = 0u - (uint32_t)(p & 1), p2 = 0u - (uint32_t)(p >> 1);
+    auto sel = [](uint32_t mask, auto x, auto y) -> uint32_t {
+        return (__builtin_bit_cast(uint32_t, x) & mask) | (__builtin_bit_cast(uint32_t, y) & ~mask);
+    };
+    Frag<TYPE> raw[FR_ROWS];
+    auto fetch = [&](int u, int ps) {
+        int m;
+        int64_t row0;
+        const uint8_t* b = unit(u, m, row0);
+        const int g = slot + 16 * ps < G ? slot + 16 * ps : G - 1;
+#pragma unroll
+        for (int r = 0; r < FR_ROWS; r++) load_frag_row(raw[r], b + (int64_t)g * (8 * BS) + r * BS, p, r);
+    };
+    const bool active = u0 + wave < u1;
+    if (active) fetch(u0 + wave, 0);
+
+    for (int ps = 0; ps < P; ps++) {
+        if (ps) __syncthreads();                 // the pass before is read out
+        // 8 loads in flight per thread and round (rows past nt read the last one again)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));            // its addresses are worked out here, not kept over the passes
+        constexpr int NLD = T * 1024 / (64 * W), LDB = 8;
+        static_assert(NLD % LDB == 0, "whole rounds of loads");
+#pragma unroll
+        for (int i0 = 0; i0 < NLD; i0 += LDB) {
+            if (i0 * 64 * W >= nt * 1024) break;
+            f32x4 v[LDB];
+#pragma unroll
+            for (int i = 0; i < LDB; i++) {
+                const int e = (i0 + i) * 64 * W + tid, t = e >> 10, c = (e >> 8 & 3) * 4 + (e & 3), l = e >> 2 & 63;
+                const int g = 16 * ps + (l >> 2) < G ? 16 * ps + (l >> 2) : G - 1;
+                v[i] = *reinterpret_cast<const f32x4_a4*>(a.x + (n0 + (t < nt ? t : nt - 1)) * a.ldx + (int64_t)g * QK + fr_elem<TYPE>(l & 3, c));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < LDB; i++) {
+                const int e = (i0 + i) * 64 * W + tid;
+                act[e >> 10][(e >> 8 & 3) * 4 + (e & 3)][e >> 2 & 63] = v[i];
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < nt * 64 * NACC; i += 64 * W) {
+            const int t = i / (64 * NACC), s = i / 64 % NACC, l = i & 63;
+            float v = 0.0f;
+            for (int c = s * (16 / NACC); c < (s + 1) * (16 / NACC); c++) {
+                const f32x4 x = act[t][c][l];
+                v = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(v, x.x), x.y), x.z), x.w);
+            }
+            sums[t][l][s] = TYPE == TYPE_Q4_K ? v : __fmul_rn(32.0f, v);
+        }
+        __syncthreads();
+        const uint32_t vmask = slot + 16 * ps < G ? 0xffffffffu : 0u;   // columns past G add +0
+        for (int u = u0 + wave; u < u1; u += W) {
+            FrRow w[FR_ROWS];
+#pragma unroll
+            for (int r = 0; r < FR_ROWS; r++) fr_unpack(w[r], prepare(raw[r], p), p);
+            int m;
+            int64_t row0;
+            unit(u, m, row0);
+            // the next unit's weights (of the next pass after the last one), in flight during this one
+            if (u + W < u1) fetch(u + W, ps);
+            else if (ps + 1 < P) fetch(u0 + wave, ps + 1);
+            const int64_t ldy = a.mg.ldy[m];
+            float* const yw = a.mg.y[m] + row0 + (lane & 3);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+            for (int t = 0; t < nt; t++) {
+                // the codes stay f16 halves in the loop: hoisted conversions would need 256 registers
+#pragma unroll
+                for (int r = 0; r < FR_ROWS; r++)
+#pragma unroll
+                    for (int c = 0; c < 32; c++) asm volatile("" : "+v"(w[r].c[c]));
+                float acc[FR_ROWS][NACC];
+#pragma unroll
+                for (int r = 0; r < FR_ROWS; r++)
+#pragma unroll
+                    for (int s = 0; s < NACC; s++) acc[r][s] = 0.0f;
+                // chunk i of the sub-blocks in turn (independent chains side by side), read FR_AHEAD chunks
+                // ahead; the barriers keep the compiler from reading all sixteen at once (64 registers)
+                auto chunk = [](int i) { return (i % NACC) * (16 / NACC) + i / NACC; };
+                float sx[NACC];
+#pragma unroll
+                for (int s = 0; s < NACC; s++) sx[s] = sums[t][lane][s];
+                f32x4 xv[FR_AHEAD + 1];
+#pragma unroll
+                for (int i = 0; i < FR_AHEAD; i++) xv[i] = act[t][chunk(i)][lane];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    if (i + FR_AHEAD < 16) xv[(i + FR_AHEAD) % (FR_AHEAD + 1)] = act[t][chunk(i + FR_AHEAD)][lane];
+                    const f32x4 v = xv[i % (FR_AHEAD + 1)];
+                    const float x[4] = {v.x, v.y, v.z, v.w};
+                    const int c = chunk(i), s = i % NACC;
+#pragma unroll
+                    for (int r = 0; r < FR_ROWS; r++)
+                        acc[r][s] = dot_halves_f32(w[r].c[2 * c], w[r].c[2 * c + 1], x, acc[r][s]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                float v[FR_ROWS];
+#pragma unroll
+                for (int r = 0; r < FR_ROWS; r++) {
+                    if constexpr (TYPE == TYPE_Q4_K) {
+                        const float plo = __fmul_rn(acc[r][0], 0x1p24f), phi = __fmul_rn(acc[r][1], 0x1p20f);
+                        const float lo = __fsub_rn(__fmul_rn(w[r].s[0], plo), __fmul_rn(w[r].s[2], sx[0]));
+                        const float hi = __fsub_rn(__fmul_rn(w[r].s[1], phi), __fmul_rn(w[r].s[3], sx[1]));
+                        v[r] = __fadd_rn(lo, hi);
+                    } else {
+                        v[r] = 0.0f;
+#pragma unroll
+                        for (int s = 0; s < 4; s++)
+                            v[r] = __fadd_rn(v[r], __fmul_rn(w[r].s[s], __fsub_rn(__fmul_rn(acc[r][s], 0x1p24f), sx[s])));
+                    }
+                    v[r] = quad_sum_f32(v[r]);
+                }
+                // lane p of each quad takes row p; the slot tree for the four rows at once
+                const uint32_t vp = sel(p2, sel(p1, v[3], v[2]), sel(p1, v[1], v[0])) & vmask;
+                const float pv = fr_slot_tree(__builtin_bit_cast(float, vp));
+                if (lane < FR_ROWS) {
+                    if constexpr (ONEPASS) yw[(n0 + t) * ldy] = __fadd_rn(pv, 0.0f);
+                    else part[(((u - u0) * FR_ROWS + lane) * nt + t) * P + ps] = pv;
+                }
+            }
+        }
+    }
+    if constexpr (ONEPASS) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < (u1 - u0) * FR_ROWS * nt; i += 64 * W) {
+        const int t = i % nt, r = i / nt % FR_ROWS, u = u0 + i / nt / FR_ROWS;
+        PassTree tr;
+        tree_init(tr);
+        for (int q = 0; q < P; q++) tree_push(tr, part[i * P + q]);
+        int m;
+        int64_t row0;
+        unit(u, m, row0);
+        a.mg.y[m][(n0 + t) * a.mg.ldy[m] + row0 + r] = tree_final(tr);
+    }
+}
+
 // ------------------------------------------------------------------ launch
 // Rows per wave: Q4_K 2 keeps per-wave register use moderate and gives many units to balance;
 // with several tokens per launch the register budget is NT*RPW <= 8 outputs per lane.  Q6_K
@@ -1202,6 +1463,68 @@ void launch_gemv_f32_group(int n, const uint8_t* const* w, const int* R, int C, 
     const uint8_t* xb = reinterpret_cast<const uint8_t*>(x);
     if (type == TYPE_Q4_K) launch3<TYPE_Q4_K, 1, 2, false, ActF32>(mg, xb, G, s);
     else launch3<TYPE_Q6_K, 1, 1, false, ActF32>(mg, xb, G, s);
+}
+
+// The rows kernel's launch: up to T rows of x per workgroup in LDS (tpg of them) and W waves, one
+// workgroup of 8 waves per CU for T = 8, two of 4 for T = 4.  tpg and the units per workgroup (k per
+// wave) are those whose rounds over the GPU take least, in the time a wave spends on one unit and one
+// row of x: per unit its tpg rows and the unpack, per workgroup the staging of tpg rows and its start.
+constexpr double FR_UNPACK = 0.9, FR_STAGE = 0.4, FR_START = 1.0;
+template <int TYPE, int T, int W>
+static void launch_f32_rows(const MatGroup& mg, int total, const float* x, int64_t ldx, int N, int G, hipStream_t s) {
+    FrArgs a{};
+    a.x = x;
+    a.ldx = ldx;
+    a.N = N;
+    a.G = G;
+    a.total_units = total;
+    a.mg = mg;
+    const int P = (G + 15) / 16, slots = device_cus() * (8 / W);
+    double best = 0;
+    for (int tpg = N < T ? N : T; tpg >= 1; tpg--) {
+        const int ntg = (N + tpg - 1) / tpg;
+        const int most = P == 1 ? 64 : FR_PART<T> / (W * FR_ROWS * tpg * P);
+        for (int k = 1; k <= most; k++) {
+            const int nrb = (total + W * k - 1) / (W * k);
+            const int64_t rounds = ((int64_t)nrb * ntg + slots - 1) / slots;
+            const double cost = rounds * (k * (tpg + FR_UNPACK) + FR_STAGE * tpg + FR_START);
+            if (a.upw == 0 || cost < best) {
+                best = cost;
+                a.upw = W * k;
+                a.nrb = nrb;
+                a.ntg = ntg;
+                a.tpg = tpg;
+            }
+        }
+    }
+    const int grid = (a.nrb + KQ_XCDS - 1) / KQ_XCDS * KQ_XCDS * a.ntg;
+    if (P == 1) hipLaunchKernelGGL((k_gemv_f32_rows<TYPE, T, W, true>), dim3(grid), dim3(64 * W), 0, s, a);
+    else hipLaunchKernelGGL((k_gemv_f32_rows<TYPE, T, W, false>), dim3(grid), dim3(64 * W), 0, s, a);
+}
+
+// fp32 activations, N >= 2 rows (row stride ldx) against n (1..3) matrices of one type.
+void launch_gemv_f32_rows(int n, const uint8_t* const* w, const int* R, int C, int type, const float* x, int64_t ldx,
+                          int N, float* const* y, const int64_t* ldy, hipStream_t s) {
+    MatGroup mg{};
+    mg.n = n;
+    int units = 0;
+    for (int i = 0; i < n; i++) {
+        mg.w[i] = w[i];
+        mg.y[i] = y[i];
+        mg.ldy[i] = ldy[i];
+        mg.first_unit[i] = units;
+        units += R[i] / FR_ROWS;
+    }
+    for (int i = n; i < 4; i++) mg.first_unit[i] = units;
+    const int G = C / QK;
+    // (T = 4 for more rows reads the weights twice as often: 24576x4096 at N = 24 113 against 169 us)
+    if (N > 4) {
+        if (type == TYPE_Q4_K) launch_f32_rows<TYPE_Q4_K, 8, 8>(mg, units, x, ldx, N, G, s);
+        else launch_f32_rows<TYPE_Q6_K, 8, 8>(mg, units, x, ldx, N, G, s);
+    } else {
+        if (type == TYPE_Q4_K) launch_f32_rows<TYPE_Q4_K, 4, 4>(mg, units, x, ldx, N, G, s);
+        else launch_f32_rows<TYPE_Q6_K, 4, 4>(mg, units, x, ldx, N, G, s);
+    }
 }
 
 }  // namespace kq

@@ -91,6 +91,10 @@ void launch_subblock_sums(const uint8_t* w, int R, int C, int type, const uint8_
 // the Q8_K GEMV with fp32 activations, one launch.
 void launch_gemv_f32_group(int n, const uint8_t* const* w, const int* R, int C, int type, const float* x,
                            float* const* y, hipStream_t s);
+// N >= 2 rows of fp32 activations (row stride ldx) against n (1..3) matrices of one type, one launch;
+// each row's outputs equal launch_gemv_f32_group on that row bit for bit.
+void launch_gemv_f32_rows(int n, const uint8_t* const* w, const int* R, int C, int type, const float* x, int64_t ldx,
+                          int N, float* const* y, const int64_t* ldy, hipStream_t s);
 void launch_dequant_rows(const uint8_t* w, int R, int C, int type, int row0, int nrows, float* y,
                          int64_t ldy, hipStream_t s);
 

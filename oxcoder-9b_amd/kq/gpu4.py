@@ -272,7 +272,13 @@ class Engine:
                 "weights": "kindi-q4-v1: Q4_K/Q6_K row tiles"}
 
     def _rows_f32(self, mats, X, outs):
-        """Mode "f32": every row of X through the fp32 GEMV (kq_gemv_multi), three matrices a launch."""
+        """Mode "f32": the rows of X through the fp32 GEMV, three matrices a call: all rows in one call
+        (kq_gemv_rows, the bits of kq_gemv_multi on each row), or row by row for 2-D outputs whose rows
+        overlap."""
+        if X.shape[0] and all(y.dim() != 2 or y.stride(0) >= R for (_, R, _, _), y in zip(mats, outs)):
+            for i in range(0, len(mats), 3):
+                ops.gemv_rows(mats[i:i + 3], X, outs[i:i + 3])
+            return 1
         for n in range(X.shape[0]):
             ys = [y[n] if y.dim() == 2 else y[n * R:(n + 1) * R] for (_, R, _, _), y in zip(mats, outs)]
             for i in range(0, len(mats), 3):

@@ -69,6 +69,29 @@ def gemv_multi(mats, x, ys):
     return ys
 
 
+def gemv_rows(mats, X, ys):
+    """Up to 3 matrices [(w, R, C, type)] on the rows of fp32 X [N][C], each output row equal to
+    gemv_multi on that row bit for bit (kq_gemv_rows); ys[i] is [N][ld_i >= R_i] or flat (rows of R_i)."""
+    n = len(mats)
+    if not 1 <= n <= 3 or len(ys) != n:
+        raise ValueError("1..3 matrices with one output each")
+    N, C_ = X.shape
+    if any(m[2] != C_ for m in mats):
+        raise ValueError("matrices sharing an input must have its column count")
+    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
+    Rs = (C.c_int * n)(*[m[1] for m in mats])
+    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    lds = [y.stride(0) if y.dim() == 2 else m[1] for m, y in zip(mats, ys)]
+    for m, y, ld in zip(mats, ys, lds):
+        if y.numel() < (N - 1) * ld + m[1]:
+            raise ValueError("output too small")
+    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
+    L = (C.c_int64 * n)(*lds)
+    _lib.check(_lib.kq().kq_gemv_rows(n, W, Rs, C_, Ts, _dev(X, "X", torch.float32), X.stride(0), N, Y, L,
+                                      _stream(mats[0][0].device)))
+    return ys
+
+
 def q8k_quantize(x, out=None):
     """x [N][C] fp32 (row stride x.stride(0)) -> Q8_K bytes uint8 [N][C/256*292]."""
     if x.dim() == 1:
