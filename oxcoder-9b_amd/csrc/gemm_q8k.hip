@@ -1041,7 +1041,8 @@ k_q8k_frag(const uint8_t* __restrict__ XQ, int M, int G, uint8_t* __restrict__ X
 }
 
 // Partial planes y_s[m][r] of the K split, added in order s = 0 .. S-1: y = ((y_0 + y_1) + y_2) + ...
-// One launch for every split matrix of a call: workgroups [blk0[j], blk0[j+1]) serve matrix j, one
+// One launch for every split matrix of a call, whatever their types (a launch per type before: the Q4_K q, k and
+// the Q6_K v of a prefill chunk paid ~4 us for the second): workgroups [blk0[j], blk0[j+1]) serve matrix j, one
 // thread per 4 consecutive outputs of a row.
 struct ReduceMat {
     const float* part;
@@ -1138,21 +1139,21 @@ size_t gemm_q8k_group_workspace(int n, const int* R, int C, int M) {
 
 size_t gemm_q8k_workspace(int R, int C, int M) { return gemm_q8k_group_workspace(1, &R, C, M); }
 
-// One reduce launch for the matrices of a group that split K.
-static void launch_reduce(const GemmGroup& gg, int M, const int* S, hipStream_t s) {
+// One reduce launch for the matrices of a call that split K (part[i] not null), whatever their types.
+static void launch_reduce(int n, const int* R, int M, float* const* y, const int64_t* ldy, float* const* part,
+                          const int* S, hipStream_t s) {
     ReduceGroup rg{};
     int blks = 0;
-    for (int i = 0; i < gg.n; i++) {
-        const GemmMat& mt = gg.m[i];
-        if (!mt.part) continue;
+    for (int i = 0; i < n; i++) {
+        if (!part[i]) continue;
         ReduceMat& rm = rg.m[rg.n++];
-        rm.part = mt.part;
-        rm.y = mt.y;
-        rm.ldy = mt.ldy;
-        rm.R = mt.R;
+        rm.part = part[i];
+        rm.y = y[i];
+        rm.ldy = ldy[i];
+        rm.R = R[i];
         rm.S = S[i];
         rm.blk0 = blks;
-        blks += (int)(((int64_t)M * (mt.R / 4) + 255) / 256);
+        blks += (int)(((int64_t)M * (R[i] / 4) + 255) / 256);
     }
     if (rg.n) hipLaunchKernelGGL(k_gemm_reduce, dim3(blks), dim3(256), 0, s, rg, M);
 }
@@ -1171,7 +1172,7 @@ static bool use_pipelined(int type, int R, int C, int M) {
 
 template <int TYPE>
 static void launch_type(const GemmGroup& gg, int wgs, int G, const uint8_t* xq, const uint8_t* xf, int M,
-                        const int* S, bool pipelined, hipStream_t s) {
+                        bool pipelined, hipStream_t s) {
     if constexpr (TYPE == TYPE_Q6_K) {          // (the Q4_K form is not dispatched: see use_pipelined)
         if (pipelined) {
             dim3 grid(wgs, (M + GP_BM - 1) / GP_BM), block(GP_THREADS);
@@ -1179,7 +1180,6 @@ static void launch_type(const GemmGroup& gg, int wgs, int G, const uint8_t* xq, 
                 hipLaunchKernelGGL((k_gemm_q8k_p<TYPE, true>), grid, block, 0, s, gg, G, xq, xf, M);
             else
                 hipLaunchKernelGGL((k_gemm_q8k_p<TYPE, false>), grid, block, 0, s, gg, G, xq, xf, M);
-            launch_reduce(gg, M, S, s);
             return;
         }
     }
@@ -1196,7 +1196,6 @@ static void launch_type(const GemmGroup& gg, int wgs, int G, const uint8_t* xq, 
         else
             hipLaunchKernelGGL((k_gemm_q8k<TYPE, GM_TN, 1, 4, false, 1>), grid, block, 0, s, gg, G, xq, xf, M);
     }
-    launch_reduce(gg, M, S, s);
 }
 
 // ------------------------------------------------------------------ the no-allocation form
@@ -1262,7 +1261,6 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
     // one launch per weight type, the matrices of that type in call order
     for (int ty : {TYPE_Q4_K, TYPE_Q6_K}) {
         GemmGroup gg{};
-        int Sg[3];
         int wgs = 0;
         for (int i = 0; i < n; i++) {
             if (type[i] != ty) continue;
@@ -1275,16 +1273,16 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
             mt.ntile = (R[i] + GM_TN - 1) / GM_TN;
             mt.gps = gps[i];
             mt.wg0 = wgs;
-            Sg[gg.n] = S[i];
             wgs += mt.ntile * S[i];
             gg.n++;
         }
         if (!gg.n) continue;
         bool pipelined = true;
         for (int i = 0; i < gg.n; i++) pipelined = pipelined && use_pipelined(ty, gg.m[i].R, C, M);
-        if (ty == TYPE_Q4_K) launch_type<TYPE_Q4_K>(gg, wgs, G, xq, ws, M, Sg, pipelined, s);
-        else launch_type<TYPE_Q6_K>(gg, wgs, G, xq, ws, M, Sg, pipelined, s);
+        if (ty == TYPE_Q4_K) launch_type<TYPE_Q4_K>(gg, wgs, G, xq, ws, M, pipelined, s);
+        else launch_type<TYPE_Q6_K>(gg, wgs, G, xq, ws, M, pipelined, s);
     }
+    launch_reduce(n, R, M, y, ldy, part, S, s);
 }
 
 static size_t q8k_rows_bytes(int C, int M) { return ((size_t)M * (C / QK) * Q8K_BYTES + 255) / 256 * 256; }
