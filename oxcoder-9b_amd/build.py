@@ -22,7 +22,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 HIP_SOURCES = ["api.hip", "q8k_quantize.hip", "producers.hip", "argmax.hip", "gemv_q8k.hip", "gemv_mfma.hip",
-               "gemv_f32.hip", "gemm_q8k.hip"]
+               "gemv_f32.hip", "gemm_q8k.hip", "gemm_small.hip"]
 HIP_FLAGS = [
     "--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -39,6 +39,7 @@ HIP_FLAGS = [
 PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 HIP_EXTRA = {"gemm_q8k.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
              "gemv_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD,
+             "gemm_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] + PRELOAD,
              "gemv_q8k.hip": PRELOAD, "q8k_quantize.hip": PRELOAD, "producers.hip": PRELOAD, "argmax.hip": PRELOAD}
 HOST_SOURCES = ["host/quantize_weights.cpp"]
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "-fopenmp", "-ffp-contract=off",

@@ -1262,8 +1262,21 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
     for (int ty : {TYPE_Q4_K, TYPE_Q6_K}) {
         GemmGroup gg{};
         int wgs = 0;
+        const uint8_t* sw[3];       // the matrices that the small kernel takes
+        int sR[3], sgps[3], ns = 0;
+        float *sy[3], *spart[3];
+        int64_t sld[3];
         for (int i = 0; i < n; i++) {
             if (type[i] != ty) continue;
+            if (gemm_small_fits(R[i], M)) {
+                sw[ns] = w[i];
+                sR[ns] = R[i];
+                sy[ns] = y[i];
+                sld[ns] = ldy[i];
+                spart[ns] = part[i];
+                sgps[ns++] = gps[i];
+                continue;
+            }
             GemmMat& mt = gg.m[gg.n];
             mt.w = w[i];
             mt.y = y[i];
@@ -1276,6 +1289,7 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
             wgs += mt.ntile * S[i];
             gg.n++;
         }
+        if (ns) launch_gemm_small_group(ns, sw, sR, C, ty, xq, ws, M, sy, sld, spart, sgps, s);
         if (!gg.n) continue;
         bool pipelined = true;
         for (int i = 0; i < gg.n; i++) pipelined = pipelined && use_pipelined(ty, gg.m[i].R, C, M);

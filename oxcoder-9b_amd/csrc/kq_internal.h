@@ -76,6 +76,14 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
 size_t gemm_f32_group_workspace(int n, const int* R, int C, int M);
 void launch_gemm_f32_group(int n, const uint8_t* const* w, const int* R, int C, const int* type, const float* x,
                            int64_t ldx, int M, float* const* y, const int64_t* ldy, uint8_t* ws, hipStream_t s);
+// The same for at most GEMM_SMALL_MAX tokens (gemm_small.hip): n (1..3) matrices of one type, one launch;
+// xf (nullable) is the fragment copy; gps: super-blocks per K split (C / 256: none), part: the split's partial
+// planes or null.  fits: whether a matrix of R rows runs it at M tokens.
+constexpr int GEMM_SMALL_MAX = 64;
+bool gemm_small_fits(int R, int M);
+void launch_gemm_small_group(int n, const uint8_t* const* w, const int* R, int C, int type, const uint8_t* xq,
+                             const uint8_t* xf, int M, float* const* y, const int64_t* ldy, float* const* part,
+                             const int* gps, hipStream_t s);
 // Device address of the static GEMM workspace on the current device (KQ_GEMM_STATIC_SCRATCH_BYTES),
 // looked up on the first call per device; fails with KQ_ERR_HIP when the lookup fails.
 int gemm_static_scratch(uint8_t** out, const char* fn);
