@@ -322,9 +322,30 @@ struct GemmGroup {
 // holds one token tile's A operands (32 VGPRs for a super-block) and uses each for both row tiles,
 // reading twice the B operands from LDS instead.  FRAG: A operands from the fragment-order copy XF,
 // else straight from the Q8_K rows XQ.
+// The matrix of this workgroup: its record's fields, picked by selects on the wave-uniform workgroup index.
+struct GemmTile {
+    const uint8_t* W;
+    float *Y, *P;
+    int64_t ldy;
+    int R, gps, split, n0;
+};
+#define KQ_GEMM_PICK(t, BN)                                                                           \
+    const int mi = nmat > 1 && bx >= wg1_ ? (nmat > 2 && bx >= wg2_ ? 2 : 1) : 0;                     \
+    auto pick = [&](auto a, auto b, auto c) { return mi == 0 ? a : mi == 1 ? b : c; };                \
+    GemmTile t;                                                                                       \
+    t.W = kq_global<const uint8_t>(pick(w0_, w1_, w2_));                                              \
+    t.Y = kq_global<float>(pick(y0_, y1_, y2_));                                                      \
+    t.P = kq_global<float>(pick(p0_, p1_, p2_));                                                      \
+    t.ldy = pick(l0_, l1_, l2_);                                                                      \
+    t.R = pick(R0_, R1_, R2_);                                                                        \
+    t.gps = pick(gp0_, gp1_, gp2_);                                                                   \
+    const int ntile = pick(nt0_, nt1_, nt2_), local = bx - pick(0, wg1_, wg2_);                       \
+    t.split = local / ntile;                                                                          \
+    t.n0 = (local - t.split * ntile) * (BN)
+
 template <int TYPE, int BN, int WN, int WM, bool FRAG, int MT>
-__global__ void __launch_bounds__(64 * WN * WM)
-k_gemm_q8k(GemmGroup gg, int G, const uint8_t* __restrict__ XQ, const uint8_t* __restrict__ XF, int M) {
+__device__ __forceinline__ void gemm_tile(const GemmTile& tl, GemmBuf<BN, 32 * MT * WM>& LB0, GemmBuf<BN, 32 * MT * WM>& LB1, int G,
+                                          const uint8_t* XQ, const uint8_t* XF, int M) {
     constexpr int BS = TYPE == TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES;
     constexpr int BM = 32 * MT * WM;
     constexpr int NTHR = 64 * WN * WM;
@@ -335,32 +356,19 @@ k_gemm_q8k(GemmGroup gg, int G, const uint8_t* __restrict__ XQ, const uint8_t* _
     constexpr int SHIFT = TYPE == TYPE_Q4_K ? 3 : 8;
     static_assert(PPR == 2 || PPR == 4, "a weight row is split in 2 or 4 parts");
     static_assert(NT * MT == 2, "two 32x32 tiles per wave");
-    __shared__ __attribute__((aligned(16))) GemmBuf<BN, BM> LB0;
-    __shared__ __attribute__((aligned(16))) GemmBuf<BN, BM> LB1;
-
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % WM, wn = wave / WM;
     const int half = lane >> 5, l32 = lane & 31;
-    // this workgroup's matrix (the argument fields picked by selects on the wave-uniform index)
-    KQ_GEMM_ARGS(gg);
-    const int mi = nmat > 1 && bx >= wg1_ ? (nmat > 2 && bx >= wg2_ ? 2 : 1) : 0;
-    auto pick = [&](auto a, auto b, auto c) { return mi == 0 ? a : mi == 1 ? b : c; };
-    const uint8_t* const W = kq_global<const uint8_t>(pick(w0_, w1_, w2_));
-    float* const Y = kq_global<float>(pick(y0_, y1_, y2_));
-    float* const P = kq_global<float>(pick(p0_, p1_, p2_));
-    const int64_t ldy = pick(l0_, l1_, l2_);
-    const int R = pick(R0_, R1_, R2_);
-    const int ntile = pick(nt0_, nt1_, nt2_);
-    const int gps = pick(gp0_, gp1_, gp2_);
-    const int local = bx - pick(0, wg1_, wg2_);
-    const int split = local / ntile;
-    const int n0 = (local - split * ntile) * BN, m0 = blockIdx.y * BM;
+    const uint8_t* const W = tl.W;
+    float* const P = tl.P;
+    const int R = tl.R, gps = tl.gps, split = tl.split;
+    const int n0 = tl.n0, m0 = blockIdx.y * BM;
     const int64_t xrow = (int64_t)G * Q8K_BYTES;
     // super-blocks [gbeg, gend) of the K split (all of them without one); with P the sums go to
     // partial plane `split` (rows of R floats) instead of Y
     const int gbeg = split * gps, gend = gbeg + gps < G ? gbeg + gps : G;
-    float* const Yo = P ? P + (int64_t)split * M * R : Y;
-    const int64_t ldo = P ? (int64_t)R : ldy;
+    float* const Yo = P ? P + (int64_t)split * M * R : tl.Y;
+    const int64_t ldo = P ? (int64_t)R : tl.ldy;
 
     // A operand of this lane for K step ks of super-block g: afrag[mt] + g * AG + ks * AK
     constexpr int AG = FRAG ? 8192 : Q8K_BYTES, AK = FRAG ? 1024 : 32;
@@ -508,6 +516,30 @@ k_gemm_q8k(GemmGroup gg, int G, const uint8_t* __restrict__ XQ, const uint8_t* _
                 if (m < M && n < R) Yo[(int64_t)m * ldo + n] = yacc[mt * NT + nt][a];
             }
         }
+}
+
+template <int TYPE, int BN, int WN, int WM, bool FRAG, int MT>
+__global__ void __launch_bounds__(64 * WN * WM)
+k_gemm_q8k(GemmGroup gg, int G, const uint8_t* __restrict__ XQ, const uint8_t* __restrict__ XF, int M) {
+    __shared__ __attribute__((aligned(16))) GemmBuf<BN, 32 * MT * WM> LB0;
+    __shared__ __attribute__((aligned(16))) GemmBuf<BN, 32 * MT * WM> LB1;
+    KQ_GEMM_ARGS(gg);
+    KQ_GEMM_PICK(t, BN);
+    gemm_tile<TYPE, BN, WN, WM, FRAG, MT>(t, LB0, LB1, G, XQ, XF, M);
+}
+
+// Both weight types in one launch: the first n6 matrices of the group are Q6_K (their longer tiles start first), the
+// others Q4_K.  For the q, k and v of a Q4_K_M layer, whose small Q6_K v alone leaves most CUs idle in a launch of its
+// own and fits into the partly filled last round of q and k's (rule and figures: mixed_types).
+template <int BN, int WN, int WM, bool FRAG, int MT>
+__global__ void __launch_bounds__(64 * WN * WM)
+k_gemm_q8k_mixed(GemmGroup gg, int n6, int G, const uint8_t* __restrict__ XQ, const uint8_t* __restrict__ XF, int M) {
+    __shared__ __attribute__((aligned(16))) GemmBuf<BN, 32 * MT * WM> LB0;
+    __shared__ __attribute__((aligned(16))) GemmBuf<BN, 32 * MT * WM> LB1;
+    KQ_GEMM_ARGS(gg);
+    KQ_GEMM_PICK(t, BN);
+    if (mi < n6) gemm_tile<TYPE_Q6_K, BN, WN, WM, FRAG, MT>(t, LB0, LB1, G, XQ, XF, M);
+    else gemm_tile<TYPE_Q4_K, BN, WN, WM, FRAG, MT>(t, LB0, LB1, G, XQ, XF, M);
 }
 
 // ------------------------------------------------------------------ pipelined kernel
@@ -1170,6 +1202,13 @@ static bool use_pipelined(int type, int R, int C, int M) {
            (int64_t)((M + GP_BM - 1) / GP_BM * GP_BM) * G * Q8K_BYTES < (int64_t(1) << 31);
 }
 
+// Whether a call's Q6_K matrices (wgs6 workgroups of 64 rows, splits included) go into one launch with its Q4_K ones:
+// when their tiles do not fill the GPU by themselves (q and k 5120x4096 Q4_K with v 1024x4096 Q6_K: 256 tokens 27.8 +
+// 16.6 us in two launches; through the 9B layer 205 -> 198 us, 777 tokens in chunks of 256 670 -> 649 us, 2048 tokens
+// 1 % faster).  Otherwise Q6_K stays in its own launch on the pipelined kernel.  Both kernels that Q6_K can run give
+// the same bits.
+static bool mixed_types(int wgs6, int M) { return (int64_t)wgs6 * ((M + GM_TM - 1) / GM_TM) < GM_FILL; }
+
 template <int TYPE>
 static void launch_type(const GemmGroup& gg, int wgs, int G, const uint8_t* xq, const uint8_t* xf, int M,
                         bool pipelined, hipStream_t s) {
@@ -1258,10 +1297,19 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
             }
         }
     }
-    // one launch per weight type, the matrices of that type in call order
-    for (int ty : {TYPE_Q4_K, TYPE_Q6_K}) {
-        GemmGroup gg{};
-        int wgs = 0;
+    // the matrices of one type in call order, and where one type's ends; Q6_K first (k_gemm_q8k_mixed)
+    GemmGroup gg{};
+    int wgs = 0, n6 = 0, wgs6 = 0;
+    auto launch_gg = [&](int ty) {
+        if (!gg.n) return;
+        bool pipelined = true;
+        for (int i = 0; i < gg.n; i++) pipelined = pipelined && use_pipelined(ty, gg.m[i].R, C, M);
+        if (ty == TYPE_Q4_K) launch_type<TYPE_Q4_K>(gg, wgs, G, xq, ws, M, pipelined, s);
+        else launch_type<TYPE_Q6_K>(gg, wgs, G, xq, ws, M, pipelined, s);
+        gg = GemmGroup{};
+        wgs = 0;
+    };
+    for (int ty : {TYPE_Q6_K, TYPE_Q4_K}) {
         const uint8_t* sw[3];       // the matrices that the small kernel takes
         int sR[3], sgps[3], ns = 0;
         float *sy[3], *spart[3];
@@ -1290,11 +1338,21 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
             gg.n++;
         }
         if (ns) launch_gemm_small_group(ns, sw, sR, C, ty, xq, ws, M, sy, sld, spart, sgps, s);
-        if (!gg.n) continue;
-        bool pipelined = true;
-        for (int i = 0; i < gg.n; i++) pipelined = pipelined && use_pipelined(ty, gg.m[i].R, C, M);
-        if (ty == TYPE_Q4_K) launch_type<TYPE_Q4_K>(gg, wgs, G, xq, ws, M, pipelined, s);
-        else launch_type<TYPE_Q6_K>(gg, wgs, G, xq, ws, M, pipelined, s);
+        if (ty == TYPE_Q6_K) {
+            n6 = gg.n;
+            wgs6 = wgs;
+            const bool both = n6 < n && mixed_types(wgs6, M);
+            if (!both) {
+                launch_gg(ty);
+                n6 = 0;
+            }
+        } else if (n6 && gg.n > n6) {
+            const dim3 grid(wgs, (M + GM_TM - 1) / GM_TM), block(256);
+            if (ws) hipLaunchKernelGGL((k_gemm_q8k_mixed<GM_TN, 1, 4, true, 1>), grid, block, 0, s, gg, n6, G, xq, ws, M);
+            else hipLaunchKernelGGL((k_gemm_q8k_mixed<GM_TN, 1, 4, false, 1>), grid, block, 0, s, gg, n6, G, xq, ws, M);
+        } else {
+            launch_gg(n6 ? TYPE_Q6_K : ty);
+        }
     }
     launch_reduce(n, R, M, y, ldy, part, S, s);
 }

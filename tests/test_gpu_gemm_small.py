@@ -43,3 +43,29 @@ def test_gemm_few_tokens(dev, orc, ty, R, C, M):
     buf = torch.empty(ops.gemm_f32_multi_workspace_bytes([m[1] for m in mats], C, M) + 256, dtype=torch.uint8, device=dev)
     ops.gemm_f32_multi(mats, dev_t(X, dev), ys, buf)
     np.testing.assert_array_equal(host(ys[0]), host(ws)[:, :R])
+
+
+@pytest.mark.parametrize("C,M,rows", [
+    (4096, 65, (4096, 1024, 1024)),             # smallest chunk of the tile kernels, K split
+    (2048, 200, (72, 1032, 8)),                 # ragged tiles
+    (512, 300, (264, 136, 5000)),               # the Q6_K part largest
+    (256, 4096, (64, 64, 1024)),                # 16 x 32 Q6_K tiles fill the GPU: launches of their own
+])
+def test_gemm_both_types_in_one_launch(dev, orc, C, M, rows):
+    """Q4_K, Q4_K and Q6_K matrices in one call, in any order: each the bits of a call of its own."""
+    print("gemm mixed", C, M, rows, flush=True)
+    mats = [(dev_t(synth(R, C, ty, 20 + i), dev), R, C, ty) for i, (R, ty) in enumerate(zip(rows, (12, 12, 14)))]
+    xqd = dev_t(orc.quantize_q8k(kqq.synthetic_activations(M, C, seed=M)), dev)
+    ref = []
+    for w, R, _, ty in mats:
+        y = torch.empty((M, R), device=dev)
+        ops.gemm_q8k(w, R, C, ty, xqd, M, y, ws=ops.gemm_workspace(R, C, M, dev))
+        ref.append(host(y))
+    for order in ((0, 1, 2), (2, 0, 1), (1, 2)):
+        sub = [mats[i] for i in order]
+        ys = [torch.full((M, m[1] + 4), -7.0, device=dev) for m in sub]
+        ws = torch.empty(ops.gemm_multi_workspace_bytes([m[1] for m in sub], C, M) + 256, dtype=torch.uint8, device=dev)
+        ops.gemm_q8k_multi(sub, xqd, M, ys, ws)
+        for i, y in zip(order, ys):
+            np.testing.assert_array_equal(host(y)[:, :rows[i]], ref[i])
+            assert np.all(host(y)[:, rows[i]:] == -7.0)
