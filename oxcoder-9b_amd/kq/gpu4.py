@@ -130,7 +130,7 @@ class Engine:
             if need:
                 self.gemm_ws = torch.empty(need + 256, dtype=torch.uint8, device=dev)
         self.argmax_ws = ops.argmax_workspace(dev)
-        self.argmax_out = torch.empty(1, dtype=torch.int32, device=dev)
+        self.argmax_out = ops.HostIndex() if torch.device(dev).type == "cuda" else None     # (None: a CPU test's Engine)
         self.logits = torch.empty(max([R for R, _ in shapes] or [1]), dtype=torch.float32, device=dev)
         self.row = torch.empty(cols, dtype=torch.float32, device=dev)     # embed / dequant output
 
@@ -239,7 +239,7 @@ class Engine:
         else:
             xq = self._quantize(x.reshape(1, -1)[:, :C], C)
             ops.gemv_q8k_argmax(w, R, C, ty, xq, y, self.argmax_ws, self.argmax_out)
-        return int(self.argmax_out.cpu()[0])
+        return self.argmax_out.read(w.device)
 
     def feed_rows(self, names, X, outs, batch_max=None):
         """Several activation rows through the named matrices, as the engine's batched prompt and
@@ -333,10 +333,12 @@ class Engine:
                                  "Engine after its weights are added, or list this group in groups=)" % (need, have))
         for m0 in range(0, M, self.chunk):
             mc = min(self.chunk, M - m0)
-            # a flat output holds rows of R
-            views = [y[m0:m0 + mc] if y.dim() == 2 else y[m0 * R:] for (_, R, _, _), y in zip(mats, outs)]
+            Xc, views = X, outs
+            if mc < M:      # a flat output holds rows of R
+                Xc = X[m0:m0 + mc]
+                views = [y[m0:m0 + mc] if y.dim() == 2 else y[m0 * R:] for (_, R, _, _), y in zip(mats, outs)]
             for i in range(0, len(mats), 3):
-                ops.gemm_f32_multi(mats[i:i + 3], X[m0:m0 + mc], views[i:i + 3], self.gemm_ws)
+                ops.gemm_f32_multi(mats[i:i + 3], Xc, views[i:i + 3], self.gemm_ws)
         return 1
 
     def embed(self, tok, out=None, name="token_embd.weight"):

@@ -6,6 +6,7 @@ launch, and a nonzero status from the library raises (ValueError for bad argumen
 HIP failures).
 """
 import ctypes as C
+import functools
 
 import torch
 
@@ -13,19 +14,29 @@ from . import _lib
 from .formats import BLOCK, Q8K_BYTES, QK, check_shape
 
 
+# Array types of 1..3 matrices' arguments, and the current stream's handle without the Stream object that
+# torch.cuda.current_stream builds: these helpers run several times per call of a few microseconds.
+_PTRS = [C.c_void_p * n for n in range(4)]
+_INTS = [C.c_int * n for n in range(4)]
+_INT64S = [C.c_int64 * n for n in range(4)]
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device):
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def _dev(t, name, dtype=None):
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise ValueError("%s must be a device tensor" % name)
     if dtype is not None and t.dtype != dtype:
         raise ValueError("%s must be %s, got %s" % (name, dtype, t.dtype))
-    if t.dim() > 0 and t.shape[-1] > 1 and t.stride(-1) != 1:
+    if t.dim() > 0 and t.stride(-1) != 1 and t.shape[-1] > 1:
         # kernels read consecutive elements of a row; rows may be strided (ld arguments)
         raise ValueError("%s must have unit stride along its last dimension" % name)
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _weights(w, R, C_, ty):
@@ -58,13 +69,13 @@ def gemv_multi(mats, x, ys):
     C_ = mats[0][2]
     if any(m[2] != C_ for m in mats) or x.numel() < C_:
         raise ValueError("matrices sharing an input must have the same column count")
-    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
-    Rs = (C.c_int * n)(*[m[1] for m in mats])
-    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    W = _PTRS[n](*[_weights(w, R, C_, ty) for (w, R, _, ty) in mats])
+    Rs = _INTS[n](*[m[1] for m in mats])
+    Ts = _INTS[n](*[m[3] for m in mats])
     for (w, R, _, ty), y in zip(mats, ys):
         if y.numel() < R:
             raise ValueError("output too small")
-    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
+    Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
     _lib.check(_lib.kq().kq_gemv_multi(n, W, Rs, C_, Ts, _dev(x, "x", torch.float32), Y, _stream(mats[0][0].device)))
     return ys
 
@@ -78,15 +89,15 @@ def gemv_rows(mats, X, ys):
     N, C_ = X.shape
     if any(m[2] != C_ for m in mats):
         raise ValueError("matrices sharing an input must have its column count")
-    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
-    Rs = (C.c_int * n)(*[m[1] for m in mats])
-    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    W = _PTRS[n](*[_weights(w, R, C_, ty) for (w, R, _, ty) in mats])
+    Rs = _INTS[n](*[m[1] for m in mats])
+    Ts = _INTS[n](*[m[3] for m in mats])
     lds = [y.stride(0) if y.dim() == 2 else m[1] for m, y in zip(mats, ys)]
     for m, y, ld in zip(mats, ys, lds):
         if y.numel() < (N - 1) * ld + m[1]:
             raise ValueError("output too small")
-    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
-    L = (C.c_int64 * n)(*lds)
+    Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
+    L = _INT64S[n](*lds)
     _lib.check(_lib.kq().kq_gemv_rows(n, W, Rs, C_, Ts, _dev(X, "X", torch.float32), X.stride(0), N, Y, L,
                                       _stream(mats[0][0].device)))
     return ys
@@ -139,10 +150,10 @@ def rms_q8k(h, w, residual=None, xn=None, xq=None):
             if (n2, d2, ld2) != (N, D, ld):
                 raise ValueError("%s must have the shape and row stride of h" % name)
     xq = _q8k_out(xq, N, D, h.device)
-    _lib.check(_lib.kq().kq_rms_q8k(C.c_void_p(h2.data_ptr()),
-                                    C.c_void_p(residual.data_ptr()) if residual is not None else None,
+    _lib.check(_lib.kq().kq_rms_q8k(h2.data_ptr(),
+                                    residual.data_ptr() if residual is not None else None,
                                     1 if residual is not None else 0, _dev(w, "w", torch.float32), D, N, ld,
-                                    C.c_void_p(xn.data_ptr()) if xn is not None else None,
+                                    xn.data_ptr() if xn is not None else None,
                                     _dev(xq, "xq", torch.uint8), _stream(h.device)))
     return xn, xq
 
@@ -157,8 +168,8 @@ def swiglu_q8k(gate, up, y=None, xq=None):
             if (n2, d2, ld2) != (N, n, ld):
                 raise ValueError("%s must have the shape and row stride of gate" % name)
     xq = _q8k_out(xq, N, n, gate.device)
-    _lib.check(_lib.kq().kq_swiglu_q8k(C.c_void_p(g2.data_ptr()), _dev(up, "up", torch.float32), n, N, ld,
-                                       C.c_void_p(y.data_ptr()) if y is not None else None,
+    _lib.check(_lib.kq().kq_swiglu_q8k(g2.data_ptr(), _dev(up, "up", torch.float32), n, N, ld,
+                                       y.data_ptr() if y is not None else None,
                                        _dev(xq, "xq", torch.uint8), _stream(gate.device)))
     return y, xq
 
@@ -178,7 +189,7 @@ def argmax(y, ws, out=None):
         raise ValueError("y must be contiguous")
     out = torch.empty(1, dtype=torch.int32, device=y.device) if out is None else out
     _lib.check(_lib.kq().kq_argmax(_dev(y, "y", torch.float32), y.numel(), _dev(ws, "ws", torch.uint8),
-                                   _dev(out, "out", torch.int32), _stream(y.device)))
+                                   _index_out(out), _stream(y.device)))
     return out
 
 
@@ -189,7 +200,7 @@ def gemv_q8k_argmax(w, R, C_, ty, xq, y, ws, out=None):
         raise ValueError("xq or y too small")
     out = torch.empty(1, dtype=torch.int32, device=w.device) if out is None else out
     _lib.check(_lib.kq().kq_gemv_q8k_argmax(pw, R, C_, ty, _dev(xq, "xq", torch.uint8), _dev(y, "y", torch.float32),
-                                            _dev(ws, "ws", torch.uint8), _dev(out, "out", torch.int32),
+                                            _dev(ws, "ws", torch.uint8), _index_out(out),
                                             _stream(w.device)))
     return out
 
@@ -217,13 +228,13 @@ def gemv_q8k_x(mats, x, ys, xq=None):
         raise ValueError("matrices sharing an input must have the same column count")
     if x.numel() < C_:
         raise ValueError("x too small")
-    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
-    Rs = (C.c_int * n)(*[m[1] for m in mats])
-    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    W = _PTRS[n](*[_weights(w, R, C_, ty) for (w, R, _, ty) in mats])
+    Rs = _INTS[n](*[m[1] for m in mats])
+    Ts = _INTS[n](*[m[3] for m in mats])
     for (w, R, _, ty), y in zip(mats, ys):
         if y.numel() < R:
             raise ValueError("output too small")
-    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
+    Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
     pq = None
     if xq is not None:
         if xq.numel() < (C_ // QK) * Q8K_BYTES:
@@ -244,17 +255,17 @@ def gemv_q8k_multi(mats, xq, N, ys):
     C_ = mats[0][2]
     if any(m[2] != C_ for m in mats):
         raise ValueError("matrices sharing an input must have the same column count")
-    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
-    Rs = (C.c_int * n)(*[m[1] for m in mats])
-    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    W = _PTRS[n](*[_weights(w, R, C_, ty) for (w, R, _, ty) in mats])
+    Rs = _INTS[n](*[m[1] for m in mats])
+    Ts = _INTS[n](*[m[3] for m in mats])
     lds = []
     for (w, R, _, ty), y in zip(mats, ys):
         ld = y.stride(0) if y.dim() == 2 else R
         if y.numel() < (N - 1) * ld + R:
             raise ValueError("output too small")
         lds.append(ld)
-    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
-    L = (C.c_int64 * n)(*lds)
+    Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
+    L = _INT64S[n](*lds)
     if xq.numel() < N * (C_ // QK) * Q8K_BYTES:
         raise ValueError("xq too small")
     _lib.check(_lib.kq().kq_gemv_q8k_multi(n, W, Rs, C_, Ts, _dev(xq, "xq", torch.uint8), N, Y, L,
@@ -318,17 +329,17 @@ def gemm_q8k_multi(mats, xq, M, ys, ws):
         raise ValueError("matrices sharing an input must have the same column count")
     if xq.numel() < M * (C_ // QK) * Q8K_BYTES:
         raise ValueError("xq too small")
-    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
-    Rs = (C.c_int * n)(*[m[1] for m in mats])
-    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    W = _PTRS[n](*[_weights(w, R, C_, ty) for (w, R, _, ty) in mats])
+    Rs = _INTS[n](*[m[1] for m in mats])
+    Ts = _INTS[n](*[m[3] for m in mats])
     lds = []
     for (w, R, _, ty), y in zip(mats, ys):
         ld = y.stride(0) if y.dim() == 2 else R
         if y.numel() < (M - 1) * ld + R:
             raise ValueError("output too small")
         lds.append(ld)
-    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
-    L = (C.c_int64 * n)(*lds)
+    Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
+    L = _INT64S[n](*lds)
     _dev(ws, "ws", torch.uint8)
     pws, nws = _aligned(ws, gemm_multi_workspace_bytes([m[1] for m in mats], C_, M))
     _lib.check(_lib.kq().kq_gemm_q8k_multi_ws(n, W, Rs, C_, Ts, _dev(xq, "xq", torch.uint8), M, Y, L, pws, nws,
@@ -336,10 +347,33 @@ def gemm_q8k_multi(mats, xq, M, ys, ws):
     return ys
 
 
+@functools.lru_cache(maxsize=4096)
+def _f32_multi_workspace(Rs, C_, M):
+    return int(_lib.kq().kq_gemm_f32_multi_workspace(len(Rs), (C.c_int * len(Rs))(*Rs), C_, M))
+
+
 def gemm_f32_multi_workspace_bytes(Rs, C_, M):
-    """Device bytes of workspace gemm_f32_multi needs (kq_gemm_f32_multi_workspace)."""
-    n = len(Rs)
-    return int(_lib.kq().kq_gemm_f32_multi_workspace(n, (C.c_int * n)(*Rs), C_, M))
+    """Device bytes of workspace gemm_f32_multi needs (kq_gemm_f32_multi_workspace, a function of these sizes alone)."""
+    return _f32_multi_workspace(tuple(Rs), C_, M)
+
+
+class HostIndex:
+    """An int32 in pinned host memory that the argmax kernels write (``out`` of argmax / gemv_q8k_argmax) and the host
+    reads after its stream: no copy back from the device (head call of 151936x4096 Q6_K: see Engine.head)."""
+
+    def __init__(self):
+        self._t = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        self._view = self._t.numpy()
+        self.ptr = self._t.data_ptr()
+
+    def read(self, device):
+        """The value, once the work on the device's current stream is done."""
+        torch.cuda.current_stream(device).synchronize()
+        return int(self._view[0])
+
+
+def _index_out(out):
+    return out.ptr if isinstance(out, HostIndex) else _dev(out, "out", torch.int32)
 
 
 def gemm_f32_multi(mats, X, ys, ws):
@@ -355,17 +389,17 @@ def gemm_f32_multi(mats, X, ys, ws):
         raise ValueError("matrices sharing an input must have its column count")
     if X.stride(1) != 1:
         raise ValueError("X needs unit stride along its rows")
-    W = (C.c_void_p * n)(*[_weights(w, R, C_, ty).value for (w, R, _, ty) in mats])
-    Rs = (C.c_int * n)(*[m[1] for m in mats])
-    Ts = (C.c_int * n)(*[m[3] for m in mats])
+    W = _PTRS[n](*[_weights(w, R, C_, ty) for (w, R, _, ty) in mats])
+    Rs = _INTS[n](*[m[1] for m in mats])
+    Ts = _INTS[n](*[m[3] for m in mats])
     lds = []
     for (w, R, _, ty), y in zip(mats, ys):
         ld = y.stride(0) if y.dim() == 2 else R
         if y.numel() < (M - 1) * ld + R:
             raise ValueError("output too small")
         lds.append(ld)
-    Y = (C.c_void_p * n)(*[_dev(y, "y", torch.float32).value for y in ys])
-    L = (C.c_int64 * n)(*lds)
+    Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
+    L = _INT64S[n](*lds)
     _dev(ws, "ws", torch.uint8)
     pws, nws = _aligned(ws, gemm_f32_multi_workspace_bytes([m[1] for m in mats], C_, M))
     _lib.check(_lib.kq().kq_gemm_f32_multi(n, W, Rs, C_, Ts, _dev(X, "X", torch.float32), X.stride(0), M, Y, L,
