@@ -294,11 +294,13 @@ int kq_gemv_q8k_multi(int n, const void* const* w, const int* R, int C, const in
     }
     if (tiles > (1 << 27)) return fail(KQ_ERR_ARG, "%s: too many rows in one call", fn);
     KQ_TRY(check_ptr(xq, 4, "xq", fn));
-    // one token over both weight types (a Q4_K_M layer's q, k and Q6_K v): one launch where possible
-    if (N == 1) {
+    // both weight types (a Q4_K_M layer's q, k and Q6_K v): one launch where possible
+    {
         const uint8_t* wa[3];
         for (int i = 0; i < n; i++) wa[i] = static_cast<const uint8_t*>(w[i]);
-        if (launch_gemv_q8k_mixed(n, wa, R, type, C, static_cast<const uint8_t*>(xq), y, as_stream(stream)))
+        const uint8_t* x8 = static_cast<const uint8_t*>(xq);
+        if (N == 1 ? launch_gemv_q8k_mixed(n, wa, R, type, C, x8, y, as_stream(stream))
+                   : launch_gemv_mfma_mixed(n, wa, R, type, C, x8, N, y, ldy, as_stream(stream)))
             return check_launch(fn);
     }
     // matrices of the same type share a launch

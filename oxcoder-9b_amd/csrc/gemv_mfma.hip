@@ -72,7 +72,7 @@ struct MvGroup {
 };
 // Kernel arguments: first, as plain scalars, what the prologue needs (the three matrices' weights, the
 // activations, the row counts, the first workgroups of matrices 1 and 2 packed as f1 | f2 << 16, and
-// NxG = N | G << 8), 13 dwords that the dispatch preloads into scalar registers
+// NxG = N | G << 8 | Q6_K matrices of a mixed launch << 16), 13 dwords that the dispatch preloads into scalar registers
 // (-amdgpu-kernarg-preload-count), so a wave's first loads wait for no argument fetch; the matrix table
 // follows for the outputs.  Matrix m's fields are picked by selects, not by an indexed load that would
 // wait for m.
@@ -80,7 +80,7 @@ struct MvGroup {
     const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, const uint8_t* __restrict__ w2,   \
         const uint8_t* __restrict__ XQ, int R0, int R1, int R2, int F12, int NxG
 #define KQ_MV_PICK(wg, rows)                                                                          \
-    const int N = NxG & 0xff, G = NxG >> 8;                                                           \
+    const int N = NxG & 0xff, G = (NxG >> 8) & 0xff;                                                  \
     const int m = (wg) >= (F12 & 0xffff) ? ((wg) >= (F12 >> 16) ? 2 : 1) : 0;                         \
     const int R = mv_pick(m, R0, R1, R2);                                                             \
     const int row0 = ((wg) - mv_pick(m, 0, F12 & 0xffff, F12 >> 16)) * (rows);                        \
@@ -522,12 +522,10 @@ __device__ __forceinline__ void buf_ld(u32x2& v, __amdgpu_buffer_rsrc_t r, int o
 
 // Workgroup and merge as k_gemv_mfma; NG groups of four tokens (N <= 4 NG) share each unpack; FP of
 // the wave's four super-blocks are in flight before the first is used.
-template <int TYPE, int NG, int LB, int FP>
-__global__ void __launch_bounds__(LB)
-k_gemv_mfma_ph(KQ_MV_HEAD, MvGroup mg) {
+template <int TYPE, int NG, int FP>
+__device__ __forceinline__ void mv_ph_tile(float (*part)[16][MV_ROWS], KQ_MV_HEAD, const MvGroup& mg) {
     typedef MvPh<TYPE> Ph;
     constexpr int BS = TYPE == TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES;
-    __shared__ float part[16][16][MV_ROWS];            // [chunk][token][row] chunk sums
     const int lane = threadIdx.x & 63;
     const int chunk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, l16 = lane & 15;
@@ -591,6 +589,14 @@ k_gemv_mfma_ph(KQ_MV_HEAD, MvGroup mg) {
     mv_merge(part, nchunks, G, N, R, row0, mv_pick(m, mg.y[0], mg.y[1], mg.y[2]), mv_pick(m, mg.ldy[0], mg.ldy[1], mg.ldy[2]));
 }
 
+#define KQ_MV_FORWARD w0, w1, w2, XQ, R0, R1, R2, F12, NxG, mg
+template <int TYPE, int NG, int LB, int FP>
+__global__ void __launch_bounds__(LB)
+k_gemv_mfma_ph(KQ_MV_HEAD, MvGroup mg) {
+    __shared__ float part[16][16][MV_ROWS];            // [chunk][token][row] chunk sums
+    mv_ph_tile<TYPE, NG, FP>(part, KQ_MV_FORWARD);
+}
+
 // ------------------------------------------------------------------ two row groups per wave
 // The plane form with each wave on two 16-row groups x two super-blocks (a "piece": half a chunk)
 // instead of one group x four: the same waves and MFMAs, but each activation operand (16 tokens x 256
@@ -601,11 +607,9 @@ k_gemv_mfma_ph(KQ_MV_HEAD, MvGroup mg) {
 // one k_gemv_mfma (and the one-token GEMV) gives.
 constexpr int MV_ROWS2 = 32;    // weight rows per workgroup of the two-group form
 
-template <int TYPE, int LB>
-__global__ void __launch_bounds__(LB)
-k_gemv_mfma_rg(KQ_MV_HEAD, MvGroup mg) {
+template <int TYPE>
+__device__ __forceinline__ void mv_rg_tile(float (*part)[16][MV_ROWS2], KQ_MV_HEAD, const MvGroup& mg) {
     constexpr int BS = TYPE == TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES;
-    __shared__ float part[16][16][MV_ROWS2];           // [piece][token][row] piece sums
     const int lane = threadIdx.x & 63;
     const int piece = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, l16 = lane & 15;
@@ -688,6 +692,35 @@ k_gemv_mfma_rg(KQ_MV_HEAD, MvGroup mg) {
     }
 }
 
+template <int TYPE, int LB>
+__global__ void __launch_bounds__(LB)
+k_gemv_mfma_rg(KQ_MV_HEAD, MvGroup mg) {
+    __shared__ float part[16][16][MV_ROWS2];           // [piece][token][row] piece sums
+    mv_rg_tile<TYPE>(part, KQ_MV_FORWARD);
+}
+
+// ------------------------------------------------------------------ both weight types in one launch
+// The q, k and v of a Q4_K_M layer share an input, and the 1024-row Q6_K v alone leaves most CUs idle for a whole
+// launch.  Here the first NxG >> 16 matrices are Q6_K (their longer workgroups start first), the others Q4_K, every
+// workgroup on the tile of its own type: the same bits as a launch per type.  With at most 16 super-blocks both types
+// have the same workgroup.  5120x4096 Q4_K with 1024x4096 Q6_K, kernel times of the two launches against the one: 4 tokens
+// 5.3 + 5.4 -> 7.8 us, 16 tokens 7.0 + 11.1 -> 10.7 us; through the 9B layers (v Q6_K in half of them) 4 / 16 tokens
+// 46.1 / 63.5 -> 43.9 / 59.9 us.
+template <bool RG, int LB>
+__global__ void __launch_bounds__(LB)
+k_gemv_mfma_mixed(KQ_MV_HEAD, MvGroup mg) {
+    __shared__ float part[16][16][RG ? MV_ROWS2 : MV_ROWS];
+    const int wg = blockIdx.x, n6 = NxG >> 16;
+    const bool q6 = wg < (n6 == 1 ? F12 & 0xffff : F12 >> 16);
+    if constexpr (RG) {
+        if (q6) mv_rg_tile<TYPE_Q6_K>(part, KQ_MV_FORWARD);
+        else mv_rg_tile<TYPE_Q4_K>(part, KQ_MV_FORWARD);
+    } else {
+        if (q6) mv_ph_tile<TYPE_Q6_K, 1, KQ_Q6P_FP1>(part, KQ_MV_FORWARD);
+        else mv_ph_tile<TYPE_Q4_K, 1, KQ_Q4P_FP1>(part, KQ_MV_FORWARD);
+    }
+}
+
 // The leading arguments of the MFMA kernels (KQ_MV_HEAD) from a group; the workgroup counts fit 16
 // bits (the dispatcher sends at most 65535 row groups to these forms).
 #define MV_HEAD_ARGS(g) (g).w[0], (g).w[1], (g).w[2], xq, (g).R[0], (g).R[1], (g).R[2], (g).first[1] | (g).first[2] << 16, N | G << 8
@@ -762,6 +795,45 @@ void launch_gemv_mfma_group(int n, const uint8_t* const* w, const int* R, int C,
     } else {
         launch_mv<TYPE_Q6_K, 1024, false, true>(mg, wgs, xq, N, G, s);
     }
+}
+
+// Whether a group of both types (rows4 / rows6 rows of each) runs as one launch: one column pass of at most 16
+// super-blocks, a Q4_K part that takes the MFMA form and a Q6_K part of fewer workgroups than the GPU has CUs (more
+// would fill it by itself).
+static bool mv_mixed_fits(int64_t rows4, int64_t rows6, int G, int N) {
+    return N >= 2 && G <= 16 && rows4 && rows6 && rows6 < 256 * MV_ROWS && (rows4 >= 4096 || N >= 4) &&
+           rows4 + rows6 < 16 * 65000;
+}
+
+bool launch_gemv_mfma_mixed(int n, const uint8_t* const* w, const int* R, const int* type, int C, const uint8_t* xq, int N,
+                            float* const* y, const int64_t* ldy, hipStream_t s) {
+    int G = C / QK, n6 = 0;
+    int64_t rows[2] = {0, 0};
+    for (int i = 0; i < n; i++) rows[type[i] == TYPE_Q6_K] += R[i];
+    if (!mv_mixed_fits(rows[0], rows[1], G, N)) return false;
+    const bool rg = N > KQ_GEMV_MFMA_Q4_PH_MAX;
+    const int wrows = rg ? MV_ROWS2 : MV_ROWS;
+    MvGroup mg{};
+    int wgs = 0, k = 0;
+    for (int ty : {TYPE_Q6_K, TYPE_Q4_K})
+        for (int i = 0; i < n; i++) {
+            if (type[i] != ty) continue;
+            mg.w[k] = w[i];
+            mg.y[k] = y[i];
+            mg.ldy[k] = ldy[i];
+            mg.R[k] = R[i];
+            mg.first[k++] = wgs;
+            wgs += (R[i] + wrows - 1) / wrows;
+            n6 += ty == TYPE_Q6_K;
+        }
+    for (int i = n; i < 4; i++) mg.first[i] = wgs;
+    G |= n6 << 8;       // in MV_HEAD_ARGS: N | G << 8 | n6 << 16
+    if (rg)
+        hipLaunchKernelGGL((k_gemv_mfma_mixed<true, 512>), dim3(wgs), dim3(64 * (((G & 0xff) + 1) / 2)), 0, s, MV_HEAD_ARGS(mg), mg);
+    else
+        hipLaunchKernelGGL((k_gemv_mfma_mixed<false, 256>), dim3(wgs), dim3(64 * (((G & 0xff) + MV_CHUNK - 1) / MV_CHUNK)), 0, s,
+                           MV_HEAD_ARGS(mg), mg);
+    return true;
 }
 
 }  // namespace kq

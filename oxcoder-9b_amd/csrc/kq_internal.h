@@ -59,6 +59,10 @@ bool launch_gemv_q8k_x_mixed(int n, const uint8_t* const* w, const int* R, const
 // Small-batch GEMV on MFMA (C <= 16384, N <= 16): rows bit-identical to the GEMV above.
 void launch_gemv_mfma_group(int n, const uint8_t* const* w, const int* R, int C, int type, const uint8_t* xq,
                             int N, float* const* y, const int64_t* ldy, hipStream_t s);
+// n (2..3) matrices of both types sharing xq, 2 <= N <= 16 tokens: one launch where that form exists (C <= 4096, few
+// Q6_K rows); false (nothing launched) otherwise.  Rows bit-identical to the groups above.
+bool launch_gemv_mfma_mixed(int n, const uint8_t* const* w, const int* R, const int* type, int C, const uint8_t* xq, int N,
+                            float* const* y, const int64_t* ldy, hipStream_t s);
 // Prefill GEMM; ws (or nullptr) holds gemm_q8k_workspace(R, C, M) bytes (256-byte aligned): the
 // activation fragments and, for grids too small to fill the GPU, the partial sums of the K split.
 size_t gemm_q8k_workspace(int R, int C, int M);
