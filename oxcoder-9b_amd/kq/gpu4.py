@@ -326,7 +326,7 @@ class Engine:
             raise ValueError("input of %d columns exceeds the engine workspace (%d)" % (C, self.max_cols))
         have = 0 if self.gemm_ws is None else self.gemm_ws.numel() - 256
         for i in range(0, len(mats), 3):
-            need = max(ops.gemm_f32_multi_workspace_bytes([m[1] for m in mats[i:i + 3]], C, mc)
+            need = max(ops.f32_multi_workspace(tuple([m[1] for m in mats[i:i + 3]]), C, mc)
                        for mc in {min(self.chunk, M), M - (M - 1) // self.chunk * self.chunk})
             if need > have:
                 raise ValueError("gemm: this call needs %d bytes of GEMM workspace, the engine holds %d (build the "

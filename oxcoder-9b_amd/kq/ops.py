@@ -347,14 +347,16 @@ def gemm_q8k_multi(mats, xq, M, ys, ws):
     return ys
 
 
-@functools.lru_cache(maxsize=4096)
-def _f32_multi_workspace(Rs, C_, M):
-    return int(_lib.kq().kq_gemm_f32_multi_workspace(len(Rs), (C.c_int * len(Rs))(*Rs), C_, M))
-
-
 def gemm_f32_multi_workspace_bytes(Rs, C_, M):
-    """Device bytes of workspace gemm_f32_multi needs (kq_gemm_f32_multi_workspace, a function of these sizes alone)."""
-    return _f32_multi_workspace(tuple(Rs), C_, M)
+    """Device bytes of workspace gemm_f32_multi needs (kq_gemm_f32_multi_workspace)."""
+    n = len(Rs)
+    return int(_lib.kq().kq_gemm_f32_multi_workspace(n, (C.c_int * n)(*Rs), C_, M))
+
+
+@functools.lru_cache(maxsize=1024)
+def f32_multi_workspace(Rs, C_, M):
+    """gemm_f32_multi_workspace_bytes of a tuple Rs, a function of these sizes alone, kept for the next call."""
+    return gemm_f32_multi_workspace_bytes(Rs, C_, M)
 
 
 class HostIndex:
@@ -401,7 +403,7 @@ def gemm_f32_multi(mats, X, ys, ws):
     Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
     L = _INT64S[n](*lds)
     _dev(ws, "ws", torch.uint8)
-    pws, nws = _aligned(ws, gemm_f32_multi_workspace_bytes([m[1] for m in mats], C_, M))
+    pws, nws = _aligned(ws, f32_multi_workspace(tuple([m[1] for m in mats]), C_, M))
     _lib.check(_lib.kq().kq_gemm_f32_multi(n, W, Rs, C_, Ts, _dev(X, "X", torch.float32), X.stride(0), M, Y, L,
                                            pws, nws, _stream(mats[0][0].device)))
     return ys
