@@ -81,9 +81,10 @@ struct MvGroup {
         const uint8_t* __restrict__ XQ, int R0, int R1, int R2, int F12, int NxG
 #define KQ_MV_PICK(wg, rows)                                                                          \
     const int N = NxG & 0xff, G = (NxG >> 8) & 0xff;                                                  \
-    const int m = (wg) >= (F12 & 0xffff) ? ((wg) >= (F12 >> 16) ? 2 : 1) : 0;                         \
+    const int f1 = F12 & 0xffff, f2 = (int)((uint32_t)F12 >> 16);                                     \
+    const int m = (wg) >= f1 ? ((wg) >= f2 ? 2 : 1) : 0;                                              \
     const int R = mv_pick(m, R0, R1, R2);                                                             \
-    const int row0 = ((wg) - mv_pick(m, 0, F12 & 0xffff, F12 >> 16)) * (rows);                        \
+    const int row0 = ((wg) - mv_pick(m, 0, f1, f2)) * (rows);                                         \
     const uint8_t* const wm = mv_pick(m, w0, w1, w2)
 template <class T> __device__ __forceinline__ T mv_pick(int m, T a, T b, T c) { return m == 0 ? a : m == 1 ? b : c; }
 
@@ -711,7 +712,7 @@ __global__ void __launch_bounds__(LB)
 k_gemv_mfma_mixed(KQ_MV_HEAD, MvGroup mg) {
     __shared__ float part[16][16][RG ? MV_ROWS2 : MV_ROWS];
     const int wg = blockIdx.x, n6 = NxG >> 16;
-    const bool q6 = wg < (n6 == 1 ? F12 & 0xffff : F12 >> 16);
+    const bool q6 = wg < (n6 == 1 ? F12 & 0xffff : (int)((uint32_t)F12 >> 16));
     if constexpr (RG) {
         if (q6) mv_rg_tile<TYPE_Q6_K>(part, KQ_MV_FORWARD);
         else mv_rg_tile<TYPE_Q4_K>(part, KQ_MV_FORWARD);

@@ -35,3 +35,17 @@ def test_mixed_types_small_batch(dev, C, rows):
         for (_, R, _, _), y, ref in zip(mats, ys, one):
             np.testing.assert_array_equal(host(y)[:, :R], ref[:N])
             assert np.all(host(y)[:, R:] == -9.0)
+
+
+def test_group_beyond_32767_workgroups(dev):
+    """A second matrix whose first workgroup number (16 rows each) needs all 16 of its bits."""
+    print("tall group", flush=True)
+    C, R0, R1, N = 256, 16 * 32776, 40, 2
+    w0 = dev_t(np.tile(synth(1024, C, 12, 1), R0 // 1024 + 1)[: R0 * 144], dev)
+    w1 = dev_t(synth(R1, C, 12, 2), dev)
+    xq = ops.q8k_quantize(dev_t(kqq.synthetic_activations(N, C, seed=N), dev))
+    y0, y1, ref = (torch.empty((N, r), device=dev) for r in (R0, R1, R1))
+    ops.gemv_q8k_multi([(w0, R0, C, 12), (w1, R1, C, 12)], xq, N, [y0, y1])
+    ops.gemv_q8k_multi([(w1, R1, C, 12)], xq, N, [ref])
+    np.testing.assert_array_equal(host(y1), host(ref))
+    np.testing.assert_array_equal(host(y0)[:, 1024:2048], host(y0)[:, :1024])
