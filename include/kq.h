@@ -121,9 +121,8 @@ int kq_gemv_q8k(const void* w, int R, int C, int type, const void* xq, int N, fl
                 int64_t ldy, void* stream);
 
 /*
- * Up to 3 matrices sharing one Q8_K input in one launch per type (q/k/v, gate/up; with one token,
- * C <= 4096 and one of the two types holding a single matrix, as a Q4_K_M layer's q, k and Q6_K v,
- * one launch for both): the Q8_K form of the CPU engine's multi-matrix gemv(m, n, A, y, x)
+ * Up to 3 matrices sharing one Q8_K input in one launch per type (q/k/v, gate/up; at C <= 4096, for a
+ * Q4_K_M layer's q, k and Q6_K v and groups like it, one launch for both): the Q8_K form of the CPU engine's multi-matrix gemv(m, n, A, y, x)
  * (kcpu4.c:100-118).  C and N are common; R[i], type[i], y[i] and ldy[i] per matrix.  Every y[i]
  * equals kq_gemv_q8k on that matrix alone bit for bit.
  */
@@ -195,7 +194,7 @@ int kq_gemm_q8k_ws(const void* w, int R, int C, int type, const void* xq, int M,
 /*
  * Up to 3 matrices sharing one Q8_K input (q/k/v, gate/up of a prefill chunk): the prefill GEMM of
  * each, with one fragment copy of the activations for all of them and one GEMM launch per weight
- * type, so the small matrices' tiles fill the GPU together.  The chunked prefill runs one GEMM per
+ * type or one for both, so the small matrices' tiles fill the GPU together.  The chunked prefill runs one GEMM per
  * projection on each chunk's shared input (chunk.py:165-177, ternary k_mm_g5q chunk.cu:820); the
  * reference's GPU operator takes several matrices on one input the same way
  * (Engine.gemv(names, x, outs), gpu4.py:95-99).  C and M are common; R[i], type[i], y[i] and

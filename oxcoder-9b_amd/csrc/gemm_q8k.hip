@@ -43,8 +43,9 @@
 // (no workspace) never splits.
 //
 // Matrices sharing the activations (q/k/v, gate/up) can go in one call: one fragment copy, and one
-// GEMM launch per weight type whose grid holds every matrix's tiles (and splits), so that small
-// matrices fill the GPU together; each matrix keeps its own split, so its results do not change.
+// GEMM launch per weight type (or one for both, k_gemm_q8k_mixed) whose grid holds every matrix's tiles
+// (and splits), so that small matrices fill the GPU together; calls of at most 64 tokens run
+// gemm_small.hip instead; each matrix keeps its own split, so its results do not change.
 #include <atomic>
 #include <mutex>
 #include <type_traits>

@@ -68,7 +68,7 @@ bool launch_gemv_mfma_mixed(int n, const uint8_t* const* w, const int* R, const 
 size_t gemm_q8k_workspace(int R, int C, int M);
 void launch_gemm_q8k(const uint8_t* w, int R, int C, int type, const uint8_t* xq, int M, float* y, int64_t ldy,
                      uint8_t* ws, hipStream_t s);
-// The same over n (1..3) matrices sharing xq: one fragment copy, one GEMM launch per weight type;
+// The same over n (1..3) matrices sharing xq: one fragment copy, one GEMM launch per weight type or one for both;
 // each matrix's results equal those of its own launch_gemm_q8k call bit for bit.
 size_t gemm_q8k_group_workspace(int n, const int* R, int C, int M);
 void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, const int* type, const uint8_t* xq,
