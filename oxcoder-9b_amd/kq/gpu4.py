@@ -130,7 +130,11 @@ class Engine:
             if need:
                 self.gemm_ws = torch.empty(need + 256, dtype=torch.uint8, device=dev)
         self.argmax_ws = ops.argmax_workspace(dev)
-        self.argmax_out = ops.HostIndex() if torch.device(dev).type == "cuda" else None     # (None: a CPU test's Engine)
+        # head's index: the pinned word its kernels write (35-70 us to allocate, so not in a call), and the tensor
+        # that argmax_out brings up to date
+        self._index = ops.HostIndex() if torch.device(dev).type == "cuda" else None
+        self._picked = None
+        self._argmax_out = torch.empty(1, dtype=torch.int32, device=dev)
         self.logits = torch.empty(max([R for R, _ in shapes] or [1]), dtype=torch.float32, device=dev)
         self.row = torch.empty(cols, dtype=torch.float32, device=dev)     # embed / dequant output
 
@@ -235,13 +239,29 @@ class Engine:
         self._check_out(y, R)
         if x.numel() < C:
             raise ValueError("head: x holds %d values, the matrix has %d columns" % (x.numel(), C))
-        if self.mode == "f32":
-            ops.gemv(w, R, C, ty, x.reshape(-1), y)
-            ops.argmax(y.reshape(-1)[:R], self.argmax_ws, self.argmax_out)
-        else:
-            xq = self._quantize(x.reshape(1, -1)[:, :C], C)
-            ops.gemv_q8k_argmax(w, R, C, ty, xq, y, self.argmax_ws, self.argmax_out)
-        return self.argmax_out.read(w.device)
+        try:
+            if self.mode == "f32":
+                ops.gemv(w, R, C, ty, x.reshape(-1), y)
+                ops.argmax(y.reshape(-1)[:R], self.argmax_ws, self._index)
+            else:
+                xq = self._quantize(x.reshape(1, -1)[:, :C], C)
+                ops.gemv_q8k_argmax(w, R, C, ty, xq, y, self.argmax_ws, self._index)
+            picked = self._index.read(w.device)
+        except BaseException:
+            # interrupted before the wait: the pinned word must not be freed while a kernel is still to write it
+            if self._index is not None:
+                self._index.read(w.device)
+            raise
+        self._picked = picked
+        return picked
+
+    @property
+    def argmax_out(self):
+        """int32[1] where the weights are: the index head picked last, and an ``out`` for ops.argmax."""
+        if self._picked is not None:
+            self._argmax_out.fill_(self._picked)
+            self._picked = None
+        return self._argmax_out
 
     def feed_rows(self, names, X, outs, batch_max=None):
         """Several activation rows through the named matrices, as the engine's batched prompt and

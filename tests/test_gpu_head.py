@@ -87,3 +87,34 @@ def test_gemv_argmax_ties_pick_the_first_row(dev, orc, ty):
     yh = y.cpu().numpy()
     top = np.flatnonzero(yh == yh.max())
     assert len(top) >= 3 and pick(out) == top[0] == orc.argmax(yh)
+
+
+@pytest.mark.parametrize("mode", ["q8k", "f32"])
+def test_engine_head_index_as_tensor_and_after_an_interrupt(dev, orc, monkeypatch, mode):
+    """argmax_out holds head's last index and serves as an ``out``; a head call that an exception leaves between its
+    launches and the wait for them returns only when they are done."""
+    from kq.gpu4 import Engine, Weights
+    R, C = 131072, 4096
+    w = Weights(dev)
+    w.add("w", torch.from_numpy(np.tile(head_matrix(1024, C, 12, seed=9), R // 1024)), R, C, 12)
+    eng = Engine(w, mode=mode, chunk=0)
+    x = dev_t(kqq.synthetic_activations(1, C, seed=8)[0], dev)
+    for i in range(2):                          # argmax_out read after every call, and after the second alone
+        tok = eng.head("w", x * (1 - 2 * i))
+        assert tok == orc.argmax(eng.logits.cpu().numpy())
+        out = eng.argmax_out
+        assert out.is_cuda and out.dtype == torch.int32 and int(out.cpu()[0]) == tok
+    y = dev_t(np.arange(100, dtype=F32), dev)
+    assert ops.argmax(y, eng.argmax_ws, eng.argmax_out) is eng.argmax_out and pick(eng.argmax_out) == 99
+
+    name = "argmax" if mode == "f32" else "gemv_q8k_argmax"
+    launch = getattr(ops, name)
+
+    def interrupted(*args):
+        launch(*args)
+        raise KeyboardInterrupt
+    monkeypatch.setattr(ops, name, interrupted)
+    torch.cuda.synchronize()
+    with pytest.raises(KeyboardInterrupt):
+        eng.head("w", x)
+    assert torch.cuda.current_stream().query()

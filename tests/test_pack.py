@@ -341,3 +341,13 @@ def test_engine_built_before_its_weights_rejects_gemm():
     w.add("m", np.zeros(16 * 144, np.uint8), 16, 256, 12)
     with pytest.raises(ValueError, match="GEMM workspace"):
         eng.gemm(["m"], torch.zeros(20, 256), [torch.empty(20, 16)])
+
+
+def test_engine_argmax_out_is_a_tensor_where_its_weights_are():
+    """The index head picked last, as a program reads it or passes it as ``out``: one int32 tensor, always the same."""
+    import torch
+    from kq.gpu4 import Engine, Weights
+    eng = Engine(Weights("cpu"))
+    out = eng.argmax_out
+    assert isinstance(out, torch.Tensor) and out.dtype == torch.int32 and out.shape == (1,)
+    assert out.device.type == "cpu" and eng.argmax_out is out
