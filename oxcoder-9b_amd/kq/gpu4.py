@@ -123,7 +123,8 @@ class Engine:
                     Cs = {self.w[n][2] for n in g}
                     if len(Cs) != 1:
                         raise ValueError("matrices of a group must share their column count")
-                    sets += [(Rs[i:i + 3], Cs.pop()) for i in range(0, len(Rs), 3)]
+                    C, = Cs
+                    sets += [(Rs[i:i + 3], C) for i in range(0, len(Rs), 3)]
             else:
                 sets = [([R, R, R], C) for R, C in shapes if C <= cols]
             need = max([self._gemm_need(Rs, C, self.chunk) for Rs, C in sets] or [0])

@@ -351,3 +351,14 @@ def test_engine_argmax_out_is_a_tensor_where_its_weights_are():
     out = eng.argmax_out
     assert isinstance(out, torch.Tensor) and out.dtype == torch.int32 and out.shape == (1,)
     assert out.device.type == "cpu" and eng.argmax_out is out
+
+
+def test_engine_sizes_a_group_of_more_than_three():
+    """gemm sends such a group three matrices at a time, and the workspace covers each part.  Host only."""
+    from kq import ops
+    from kq.gpu4 import Engine, Weights
+    w = Weights("cpu")
+    for name, R in (("a", 16), ("b", 8), ("c", 8), ("d", 2048)):
+        w.add(name, np.zeros(R * 2 * 144, np.uint8), R, 512, 12)
+    need = max(ops.gemm_f32_multi_workspace_bytes(Rs, 512, m) for Rs in ([16, 8, 8], [2048]) for m in range(1, 257))
+    assert Engine(w, groups=[list("abcd")], chunk=256).gemm_ws.numel() == need + 256
