@@ -296,13 +296,15 @@ class Engine:
 
     def _rows_f32(self, mats, X, outs):
         """Mode "f32": the rows of X through the fp32 GEMV, three matrices a call: all rows in one call
-        (kq_gemv_rows, the bits of kq_gemv_multi on each row), or row by row for 2-D outputs whose rows
-        overlap."""
-        if X.shape[0] and all(y.dim() != 2 or y.stride(0) >= R for (_, R, _, _), y in zip(mats, outs)):
+        (kq_gemv_rows, the bits of kq_gemv_multi on each row), or row by row, with that call's checks, for
+        outputs that are not flat or N whole rows apart from one another."""
+        N = X.shape[0]
+        if N and all(y.dim() == 1 or y.dim() == 2 and y.shape[0] >= N and min(y.shape[1], y.stride(0)) >= R
+                     for (_, R, _, _), y in zip(mats, outs)):
             for i in range(0, len(mats), 3):
                 ops.gemv_rows(mats[i:i + 3], X, outs[i:i + 3])
             return 1
-        for n in range(X.shape[0]):
+        for n in range(N):
             ys = [y[n] if y.dim() == 2 else y[n * R:(n + 1) * R] for (_, R, _, _), y in zip(mats, outs)]
             for i in range(0, len(mats), 3):
                 ops.gemv_multi(mats[i:i + 3], X[n], ys[i:i + 3])

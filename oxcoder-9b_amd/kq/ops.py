@@ -94,7 +94,8 @@ def gemv_rows(mats, X, ys):
     Ts = _INTS[n](*[m[3] for m in mats])
     lds = [y.stride(0) if y.dim() == 2 else m[1] for m, y in zip(mats, ys)]
     for m, y, ld in zip(mats, ys, lds):
-        if y.numel() < (N - 1) * ld + m[1]:
+        # a view narrower than R may hold enough elements in all, but its rows do not hold R
+        if y.numel() < (N - 1) * ld + m[1] or y.dim() == 2 and (y.shape[0] < N or y.shape[1] < m[1]):
             raise ValueError("output too small")
     Y = _PTRS[n](*[_dev(y, "y", torch.float32) for y in ys])
     L = _INT64S[n](*lds)

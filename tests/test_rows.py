@@ -59,3 +59,29 @@ def test_rows_argument_errors(N, ldx, ldy, msg):
     P, I, L = ctypes.c_void_p * 1, ctypes.c_int * 1, ctypes.c_int64 * 1
     rc = lib.kq_gemv_rows(1, P(4096), I(64), 256, I(12), ctypes.c_void_p(4096), ldx, N, P(8192), L(ldy), None)
     assert rc == _lib.KQ_ERR_ARG and msg in lib.kq_last_error().decode()
+
+
+@pytest.mark.gpu
+def test_rows_refuse_views_narrower_than_the_matrix(dev):
+    """A column view of fewer than R values a row holds enough elements once it has rows to spare, and its stride is
+    wide enough: the call is refused, as one row at a time is, and the columns beside the view stay as they were."""
+    from kq.gpu4 import Engine, Weights
+    R, C, N = 200, 256, 3
+    w = Weights(dev)
+    w.add("m", kqq.synthetic_matrix(R, C, 12, seed=1), R, C, 12)
+    eng = Engine(w, mode="f32", chunk=0)
+    X = torch.from_numpy(kqq.synthetic_activations(N, C, seed=2)).to(dev)
+    base = torch.full((10, 300), -5.0, device=dev)
+    for y, err in ((base[:, :100], ValueError), (base.clone().as_strided((2, 300), (200, 1)), IndexError)):
+        with pytest.raises(ValueError):                  # (the second: elements for three rows, but two of them)
+            ops.gemv_rows([w["m"]], X, [y])
+        with pytest.raises(err):
+            eng.gemv_batch(["m"], X, [y])
+    assert (base == -5.0).all()
+    ref, got = torch.empty((N, R), device=dev), torch.full((N, 300), -5.0, device=dev)
+    eng.gemv_batch(["m"], X, [ref])
+    eng.gemv_batch(["m"], X, [got])                      # rows wider than R
+    assert torch.equal(got[:, :R], ref) and (got[:, R:] == -5.0).all()
+    cube = torch.empty((1, 1, R), device=dev)
+    eng.gemv_batch(["m"], X[:1], [cube])                 # any shape that holds one row
+    assert torch.equal(cube.view(R), ref[0])
