@@ -907,14 +907,16 @@ k_gemv_q8k_split2(KQ_GEMV_HEAD, int nwgA, MatGroup mgA, MatGroup mgB, uint8_t* x
 // row: 256 of the ~350 VALU instructions a wave spends per unit and row of x.  The lanes' sums of four
 // weight rows go through one slot tree (fr_slot_tree).  Each activation read from LDS serves FR_ROWS
 // rows.  Measured, one-row launches -> this kernel, us: 24576x4096 Q4_K at N = 2 / 5 28.9 / 69.8 -> 18.7
-// / 30.9, at N = 24 113 (61 for the multiply-adds alone at 2.4 GHz); 4096x12288 Q6_K at N = 2 / 5 25.2 /
-// 60.3 -> 22.6 / 31.1; 1024x4096 Q4_K at N = 2 8.9 -> 4.9: faster at every size from two rows on.  A
+// / 30.9, at N = 24 113 (61 for the multiply-adds alone at 2.4 GHz); 4096x12288 Q6_K at N = 2 / 5 26.0 /
+// 61.5 -> 21.5 / 29.5; 1024x4096 Q4_K at N = 2 8.9 -> 4.9: faster at every size from two rows on.  A
 // 24-row prompt through the 9B layer 1330 -> 260.
 constexpr int FR_ROWS = 4;                  // weight rows per unit
-#ifndef KQ_FR_AHEAD
-#define KQ_FR_AHEAD 3
-#endif
-constexpr int FR_AHEAD = KQ_FR_AHEAD;       // activation chunks read ahead of their use
+// Activation chunks read ahead of their use: three for Q4_K; one for Q6_K, whose raw blocks and codes leave no
+// registers for more.  With three, and the factors of the sub-block sums and the lane masks kept over the
+// multiply-adds, it spilled 22 registers in the loop over the rows of x: 4096x12288 at N = 2 / 5 / 8 / 24
+// 23.8 / 32.4 / 37.4 / 80 -> 21.5 / 29.5 / 33.9 / 77 us, 1024x4096 7.2 / 9.6 / 10.3 / 13.6 -> 6.6 / 8.3 / 8.4 / 12.0,
+// 24576x4096 at N = 24 unchanged (132); with two it spilled 4 and lay between.
+template <int TYPE> constexpr int FR_AHEAD = TYPE == TYPE_Q4_K ? 3 : 1;
 template <int T> constexpr int FR_PART = 512 * T;   // floats of pass values a workgroup holds (several column passes)
 
 // One weight row's quarter of a super-block, unpacked: c[] holds the codes as f16 halves in the order
@@ -990,7 +992,8 @@ __global__ void __launch_bounds__(64 * W, 2)
 k_gemv_f32_rows(FrArgs a) {
     constexpr int BS = TYPE == TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES;
     constexpr int WPT = 8 / FR_ROWS;
-    constexpr int NACC = FR_NACC<TYPE>;
+    constexpr int NACC = FR_NACC<TYPE>, AHEAD = FR_AHEAD<TYPE>;
+    constexpr bool LEAN = TYPE == TYPE_Q6_K;     // registers are short: see FR_AHEAD
     // [token][chunk][lane]: a wave's read of one chunk is one contiguous 1 KB
     __shared__ f32x4 act[T][16][64];
     __shared__ float sums[T][64][NACC];          // Q4_K: sums of the two sub-blocks; Q6_K: 32 * sum of each
@@ -1012,8 +1015,7 @@ k_gemv_f32_rows(FrArgs a) {
         row0 = (int64_t)v * FR_ROWS;
         return a.mg.w[m] + (int64_t)(v / WPT) * G * (8 * BS) + (v % WPT) * FR_ROWS * BS;
     };
-    // bit selects (conditional expressions became branches)
-    const uint32_t p1 = 0u - (uint32_t)(p & 1), p2 = 0u - (uint32_t)(p >> 1);
+    // bit select (conditional expressions became branches)
     auto sel = [](uint32_t mask, auto x, auto y) -> uint32_t {
         return (__builtin_bit_cast(uint32_t, x) & mask) | (__builtin_bit_cast(uint32_t, y) & ~mask);
     };
@@ -1064,7 +1066,6 @@ k_gemv_f32_rows(FrArgs a) {
             sums[t][l][s] = TYPE == TYPE_Q4_K ? v : __fmul_rn(32.0f, v);
         }
         __syncthreads();
-        const uint32_t vmask = slot + 16 * ps < G ? 0xffffffffu : 0u;   // columns past G add +0
         for (int u = u0 + wave; u < u1; u += W) {
             FrRow w[FR_ROWS];
 #pragma unroll
@@ -1090,19 +1091,23 @@ k_gemv_f32_rows(FrArgs a) {
                 for (int r = 0; r < FR_ROWS; r++)
 #pragma unroll
                     for (int s = 0; s < NACC; s++) acc[r][s] = 0.0f;
-                // chunk i of the sub-blocks in turn (independent chains side by side), read FR_AHEAD chunks
+                // chunk i of the sub-blocks in turn (independent chains side by side), read AHEAD chunks
                 // ahead; the barriers keep the compiler from reading all sixteen at once (64 registers)
                 auto chunk = [](int i) { return (i % NACC) * (16 / NACC) + i / NACC; };
                 float sx[NACC];
+                auto load_sx = [&]() {
 #pragma unroll
-                for (int s = 0; s < NACC; s++) sx[s] = sums[t][lane][s];
-                f32x4 xv[FR_AHEAD + 1];
+                    for (int s = 0; s < NACC; s++) sx[s] = sums[t][lane][s];
+                };
+                if constexpr (!LEAN) load_sx();
+                f32x4 xv[AHEAD + 1];
 #pragma unroll
-                for (int i = 0; i < FR_AHEAD; i++) xv[i] = act[t][chunk(i)][lane];
+                for (int i = 0; i < AHEAD; i++) xv[i] = act[t][chunk(i)][lane];
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    if (i + FR_AHEAD < 16) xv[(i + FR_AHEAD) % (FR_AHEAD + 1)] = act[t][chunk(i + FR_AHEAD)][lane];
-                    const f32x4 v = xv[i % (FR_AHEAD + 1)];
+                    if (i + AHEAD < 16) xv[(i + AHEAD) % (AHEAD + 1)] = act[t][chunk(i + AHEAD)][lane];
+                    else if (LEAN && i + AHEAD == 16) load_sx();    // in the first chunk's registers that are free
+                    const f32x4 v = xv[i % (AHEAD + 1)];
                     const float x[4] = {v.x, v.y, v.z, v.w};
                     const int c = chunk(i), s = i % NACC;
 #pragma unroll
@@ -1127,6 +1132,10 @@ k_gemv_f32_rows(FrArgs a) {
                     v[r] = quad_sum_f32(v[r]);
                 }
                 // lane p of each quad takes row p; the slot tree for the four rows at once
+                int ln = lane;
+                if constexpr (LEAN) asm volatile("" : "+v"(ln));    // masks worked out here, not kept over the loop
+                const uint32_t p1 = 0u - (uint32_t)(ln & 1), p2 = 0u - (uint32_t)(ln >> 1 & 1);
+                const uint32_t vmask = (ln >> 2) + 16 * ps < G ? 0xffffffffu : 0u;   // columns past G add +0
                 const uint32_t vp = sel(p2, sel(p1, v[3], v[2]), sel(p1, v[1], v[0])) & vmask;
                 const float pv = fr_slot_tree(__builtin_bit_cast(float, vp));
                 if (lane < FR_ROWS) {

@@ -316,3 +316,12 @@ def test_gemv_q8k_x_argument_errors(n, C, x, xq, msg):
     rc = lib.kq_gemv_q8k_x(n, W, R, C, T, ctypes.c_void_p(x), Y, None if xq is None else ctypes.c_void_p(xq), None)
     assert rc == _lib.KQ_ERR_ARG
     assert msg in lib.kq_last_error().decode()
+
+
+def test_no_kernel_spills():
+    """Every kernel's metadata (MessagePack in libkq.so) gives 0 bytes of scratch per lane: nothing spills."""
+    blob = open(os.path.join(ROOT, "oxcoder-9b_amd", "kq", "libkq.so"), "rb").read()
+    names = re.findall(rb"\xa5\.name(?:[\xa0-\xbf]|\xd9.|\xda..)(_ZN2kq\w+)", blob, re.S)
+    scratch = [m.end() for m in re.finditer(rb"\xbb\.private_segment_fixed_size", blob)]
+    assert len(names) == len(scratch) > 50
+    assert [n.decode() for n, at in zip(names, scratch) if blob[at] != 0] == []
