@@ -908,8 +908,8 @@ k_gemv_q8k_split2(KQ_GEMV_HEAD, int nwgA, MatGroup mgA, MatGroup mgB, uint8_t* x
 // weight rows go through one slot tree (fr_slot_tree).  Each activation read from LDS serves FR_ROWS
 // rows.  Measured, one-row launches -> this kernel, us: 24576x4096 Q4_K at N = 2 / 5 28.9 / 69.8 -> 18.7
 // / 30.9, at N = 24 113 (61 for the multiply-adds alone at 2.4 GHz); 4096x12288 Q6_K at N = 2 / 5 26.0 /
-// 61.5 -> 21.5 / 29.5; 1024x4096 Q4_K at N = 2 8.9 -> 4.9: faster at every size from two rows on.  A
-// 24-row prompt through the 9B layer 1330 -> 260.
+// 61.5 -> 21.5 / 29.5; 1024x4096 Q4_K at N = 2 9.7 -> 5.4: faster from two rows on but for
+// some short, wide Q6_K matrices (f32_row_by_row).  A 24-row prompt through the 9B layer 1330 -> 254.
 constexpr int FR_ROWS = 4;                  // weight rows per unit
 // Activation chunks read ahead of their use: three for Q4_K; one for Q6_K, whose raw blocks and codes leave no
 // registers for more.  With three, and the factors of the sub-block sums and the lane masks kept over the
@@ -1511,6 +1511,19 @@ static void launch_f32_rows(const MatGroup& mg, int total, const float* x, int64
     else hipLaunchKernelGGL((k_gemv_f32_rows<TYPE, T, W, false>), dim3(grid), dim3(64 * W), 0, s, a);
 }
 
+// Whether N rows of x go through the one-row kernel, a launch each: two or three rows against a short, wide Q6_K
+// matrix (or a group of `rows` rows in all).  From 5 column passes on that kernel gives each of up to 1024 rows a wave that
+// walks the passes with no barrier, where a workgroup of the rows kernel stages every pass behind two; more rows than
+// that take the one-row kernel a second round.  Graph replays, us, rows kernel against one-row launches: 64x28672 at
+// N = 2 28.5 / 19.6, 1024x16640 22.6 / 18.7, 1024x61440 60.5 / 51.3 (1280x61440 61.6 / 93.9); at N = 3 64x45056 43.7 /
+// 40.7 and 16x61440 58.0 / 52.4 (128x45056 43.9 / 44.8; 8x45056, half a workgroup, 39.2 / 39.9).  At fewer columns the two
+// are within 2 %, and with more rows of x and for Q4_K, whose one-row waves hold two rows (64x28672 at N = 2 22.9 /
+// 37.5), the rows kernel is the faster.
+static bool f32_row_by_row(int type, int rows, int G, int N) {
+    if (type != TYPE_Q6_K) return false;
+    return N == 2 ? G > 64 && rows <= 1024 : N == 3 && G > 128 && rows >= 16 && rows <= 64;
+}
+
 // fp32 activations, N >= 2 rows (row stride ldx) against n (1..3) matrices of one type.
 void launch_gemv_f32_rows(int n, const uint8_t* const* w, const int* R, int C, int type, const float* x, int64_t ldx,
                           int N, float* const* y, const int64_t* ldy, hipStream_t s) {
@@ -1526,6 +1539,14 @@ void launch_gemv_f32_rows(int n, const uint8_t* const* w, const int* R, int C, i
     }
     for (int i = n; i < 4; i++) mg.first_unit[i] = units;
     const int G = C / QK;
+    if (f32_row_by_row(type, units * FR_ROWS, G, N)) {
+        for (int r = 0; r < N; r++) {
+            float* yr[3];
+            for (int i = 0; i < n; i++) yr[i] = y[i] + r * ldy[i];
+            launch_gemv_f32_group(n, w, R, C, type, x + r * ldx, yr, s);
+        }
+        return;
+    }
     // (T = 4 for more rows reads the weights twice as often: 24576x4096 at N = 24 113 against 169 us)
     if (N > 4) {
         if (type == TYPE_Q4_K) launch_f32_rows<TYPE_Q4_K, 8, 8>(mg, units, x, ldx, N, G, s);

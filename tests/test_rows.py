@@ -17,6 +17,10 @@ from kq import quantize as kqq
     ((136, 24), 4096, (12, 12), 4), ((264, 40, 8), 4096, (12, 14, 12), 9), ((2056, 512, 512), 4096, (12, 12, 14), 24),
     ((40,), 4352, (14,), 3), ((72,), 12288, (12,), 8), ((264,), 12288, (14,), 17), ((24,), 17408, (12,), 6),
     ((16,), 61440, (14,), 11), ((16,), 61440, (12,), 4),
+    # two and three rows against short, wide Q6_K matrices: either side of the lines where they go row by row
+    ((512, 512), 16640, (14, 14), 2), ((1032,), 16640, (14,), 2), ((1024,), 16384, (14,), 2),
+    ((64, 8), 33024, (14, 12), 3), ((72,), 33024, (14,), 3), ((64,), 32768, (14,), 3), ((8,), 61440, (14,), 3),
+    ((16,), 61440, (14,), 3), ((8,), 61440, (14,), 2),
 ])
 def test_rows_equal_one_row_calls(dev, Rs, C, types, N):
     mats = [(torch.from_numpy(kqq.synthetic_matrix(R, C, t, seed=R + i)).to(dev), R, C, t)
