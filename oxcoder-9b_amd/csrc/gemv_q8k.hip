@@ -1506,7 +1506,14 @@ static void launch_f32_rows(const MatGroup& mg, int total, const float* x, int64
             }
         }
     }
-    const int grid = (a.nrb + KQ_XCDS - 1) / KQ_XCDS * KQ_XCDS * a.ntg;
+    const int64_t grid = (int64_t)((a.nrb + KQ_XCDS - 1) / KQ_XCDS * KQ_XCDS) * a.ntg;
+    if (N > 1 && grid * (64 * W) >= (int64_t)1 << 32) {     // more threads than a launch takes: the rows of x in two parts
+        const int h = N / 2;
+        launch_f32_rows<TYPE, T, W>(mg, total, x, ldx, h, G, s);
+        for (int i = 0; i < mg.n; i++) a.mg.y[i] += h * mg.ldy[i];
+        launch_f32_rows<TYPE, T, W>(a.mg, total, x + h * ldx, ldx, N - h, G, s);
+        return;
+    }
     if (P == 1) hipLaunchKernelGGL((k_gemv_f32_rows<TYPE, T, W, true>), dim3(grid), dim3(64 * W), 0, s, a);
     else hipLaunchKernelGGL((k_gemv_f32_rows<TYPE, T, W, false>), dim3(grid), dim3(64 * W), 0, s, a);
 }

@@ -89,3 +89,20 @@ def test_rows_refuse_views_narrower_than_the_matrix(dev):
     cube = torch.empty((1, 1, R), device=dev)
     eng.gemv_batch(["m"], X[:1], [cube])                 # any shape that holds one row
     assert torch.equal(cube.view(R), ref[0])
+
+
+@pytest.mark.gpu
+def test_rows_beyond_one_launch(dev):
+    """More rows of x than one launch has threads for (2^32 at 8 rows a workgroup of 512): every row is written, and
+    those around the parts' edges have the one-row call's bits.  The rows of x overlap, each one float further on."""
+    R, C, N = 8, 256, (1 << 23) + 5
+    mat = (torch.from_numpy(kqq.synthetic_matrix(R, C, 12, seed=4)).to(dev), R, C, 12)
+    base = torch.randn(N + C, generator=torch.Generator(device=dev).manual_seed(1), device=dev)
+    X = base.as_strided((N, C), (1, 1))
+    y = torch.full((N, R), float("nan"), device=dev)
+    ops.gemv_rows([mat], X, [y])
+    assert not y.isnan().any()
+    for n in (0, 1, N // 4, N // 2 - 1, N // 2, N // 2 + 1, N - 9, N - 1):
+        want = torch.empty(R, device=dev)
+        ops.gemv_multi([mat], X[n], [want])
+        assert torch.equal(y[n], want), n
