@@ -318,11 +318,6 @@ struct GemmGroup {
                  "+s"(nmat) : "s"(G), "s"(XQ), "s"(XF), "s"(M));                                     \
     __builtin_amdgcn_sched_barrier(0)
 
-// WN waves along n times WM along m; each wave owns MT token tiles x NT = 2/MT weight-row tiles of
-// 32x32 (two MFMA tiles), the workgroup BM = 32*MT*WM tokens x BN = 32*NT*WN rows.  With MT = 1 a wave
-// holds one token tile's A operands (32 VGPRs for a super-block) and uses each for both row tiles,
-// reading twice the B operands from LDS instead.  FRAG: A operands from the fragment-order copy XF,
-// else straight from the Q8_K rows XQ.
 // The matrix of this workgroup: its record's fields, picked by selects on the wave-uniform workgroup index.
 struct GemmTile {
     const uint8_t* W;
@@ -344,6 +339,11 @@ struct GemmTile {
     t.split = local / ntile;                                                                          \
     t.n0 = (local - t.split * ntile) * (BN)
 
+// WN waves along n times WM along m; each wave owns MT token tiles x NT = 2/MT weight-row tiles of
+// 32x32 (two MFMA tiles), the workgroup BM = 32*MT*WM tokens x BN = 32*NT*WN rows.  With MT = 1 a wave
+// holds one token tile's A operands (32 VGPRs for a super-block) and uses each for both row tiles,
+// reading twice the B operands from LDS instead.  FRAG: A operands from the fragment-order copy XF,
+// else straight from the Q8_K rows XQ.
 template <int TYPE, int BN, int WN, int WM, bool FRAG, int MT>
 __device__ __forceinline__ void gemm_tile(const GemmTile& tl, GemmBuf<BN, 32 * MT * WM>& LB0, GemmBuf<BN, 32 * MT * WM>& LB1, int G,
                                           const uint8_t* XQ, const uint8_t* XF, int M) {
@@ -532,15 +532,16 @@ k_gemm_q8k(GemmGroup gg, int G, const uint8_t* __restrict__ XQ, const uint8_t* _
 // Both weight types in one launch: the first n6 matrices of the group are Q6_K (their longer tiles start first), the
 // others Q4_K.  For the q, k and v of a Q4_K_M layer, whose small Q6_K v alone leaves most CUs idle in a launch of its
 // own and fits into the partly filled last round of q and k's (rule and figures: mixed_types).
-template <int BN, int WN, int WM, bool FRAG, int MT>
+// Always from the fragment copy: a call without a workspace has one matrix.
+template <int BN, int WN, int WM, int MT>
 __global__ void __launch_bounds__(64 * WN * WM)
 k_gemm_q8k_mixed(GemmGroup gg, int n6, int G, const uint8_t* __restrict__ XQ, const uint8_t* __restrict__ XF, int M) {
     __shared__ __attribute__((aligned(16))) GemmBuf<BN, 32 * MT * WM> LB0;
     __shared__ __attribute__((aligned(16))) GemmBuf<BN, 32 * MT * WM> LB1;
     KQ_GEMM_ARGS(gg);
     KQ_GEMM_PICK(t, BN);
-    if (mi < n6) gemm_tile<TYPE_Q6_K, BN, WN, WM, FRAG, MT>(t, LB0, LB1, G, XQ, XF, M);
-    else gemm_tile<TYPE_Q4_K, BN, WN, WM, FRAG, MT>(t, LB0, LB1, G, XQ, XF, M);
+    if (mi < n6) gemm_tile<TYPE_Q6_K, BN, WN, WM, true, MT>(t, LB0, LB1, G, XQ, XF, M);
+    else gemm_tile<TYPE_Q4_K, BN, WN, WM, true, MT>(t, LB0, LB1, G, XQ, XF, M);
 }
 
 // ------------------------------------------------------------------ pipelined kernel
@@ -1342,15 +1343,14 @@ void launch_gemm_q8k_group(int n, const uint8_t* const* w, const int* R, int C, 
         if (ty == TYPE_Q6_K) {
             n6 = gg.n;
             wgs6 = wgs;
-            const bool both = n6 < n && mixed_types(wgs6, M);
+            const bool both = ws && n6 < n && mixed_types(wgs6, M);
             if (!both) {
                 launch_gg(ty);
                 n6 = 0;
             }
         } else if (n6 && gg.n > n6) {
             const dim3 grid(wgs, (M + GM_TM - 1) / GM_TM), block(256);
-            if (ws) hipLaunchKernelGGL((k_gemm_q8k_mixed<GM_TN, 1, 4, true, 1>), grid, block, 0, s, gg, n6, G, xq, ws, M);
-            else hipLaunchKernelGGL((k_gemm_q8k_mixed<GM_TN, 1, 4, false, 1>), grid, block, 0, s, gg, n6, G, xq, ws, M);
+            hipLaunchKernelGGL((k_gemm_q8k_mixed<GM_TN, 1, 4, 1>), grid, block, 0, s, gg, n6, G, xq, ws, M);
         } else {
             launch_gg(n6 ? TYPE_Q6_K : ty);
         }
