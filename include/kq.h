@@ -73,7 +73,9 @@ int kq_gemv_multi(int n, const void* const* w, const int* R, int C, const int* t
  * floats, at least R[i]), each equal to kq_gemv_multi on that row bit for bit.  The fp32 form of the
  * batched layout y[ntok][R] (tc.cu:306-310): prompts and drafted tokens in the reference's own
  * numerics, which the reference's Q4 engine feeds token by token (gpu4.py:109-110), with the weights
- * read and unpacked once per 8 rows instead of once per row.  One launch per weight type.
+ * read and unpacked once per group of up to 8 rows (the launch picks the group) instead of once per row.
+ * One launch per weight type; two or three rows against a short, wide Q6_K matrix a launch each, and
+ * more rows than one launch has threads for (millions) several.
  */
 int kq_gemv_rows(int n, const void* const* w, const int* R, int C, const int* type, const float* x, int64_t ldx,
                  int N, float* const* y, const int64_t* ldy, void* stream);
@@ -121,9 +123,11 @@ int kq_gemv_q8k(const void* w, int R, int C, int type, const void* xq, int N, fl
                 int64_t ldy, void* stream);
 
 /*
- * Up to 3 matrices sharing one Q8_K input in one launch per type (q/k/v, gate/up; at C <= 4096, for a
- * Q4_K_M layer's q, k and Q6_K v and groups like it, one launch for both): the Q8_K form of the CPU engine's multi-matrix gemv(m, n, A, y, x)
- * (kcpu4.c:100-118).  C and N are common; R[i], type[i], y[i] and ldy[i] per matrix.  Every y[i]
+ * Up to 3 matrices sharing one Q8_K input in one launch per type (q/k/v, gate/up), or, at C <= 4096, in
+ * one for both types (a Q4_K_M layer's q, k and Q6_K v): with one token when one of the types holds a
+ * single matrix, with more when the Q6_K matrices have fewer than 4096 rows in all and the Q4_K ones at
+ * least 4096 (or any number from 4 tokens on).  The Q8_K form of the CPU engine's multi-matrix
+ * gemv(m, n, A, y, x) (kcpu4.c:100-118).  C and N are common; R[i], type[i], y[i] and ldy[i] per matrix.  Every y[i]
  * equals kq_gemv_q8k on that matrix alone bit for bit.
  */
 int kq_gemv_q8k_multi(int n, const void* const* w, const int* R, int C, const int* type, const void* xq,

@@ -110,7 +110,7 @@ class Engine:
         dev = self.device
         # Q8_K workspace (the reference's reused xp scratch, gpu4.py:70-79)
         self.xq = torch.empty(self.max_rows * (cols // QK) * Q8K_BYTES, dtype=torch.uint8, device=dev)
-        # prefill GEMM workspace (mode "q8k" only: "f32" prefills row by row): the most any chunk
+        # prefill GEMM workspace (mode "q8k" only: "f32" runs the fp32 GEMV's rows): the most any chunk
         # (1..chunk rows) of the matrix groups gemm will see needs.  With ``groups`` (lists of names
         # that share an input, e.g. [q, k, v], [gate, up]) it is sized for those, three at a time as
         # gemm sends them; without, for any three matrices of one shape (which bounds every mix).
@@ -230,8 +230,8 @@ class Engine:
         then the argmax over the logits (gemv([head]) + k_argmax, engine.py:326-328; kq_gemv then
         kq_argmax).  Mode "q8k" quantizes x and the GEMV finds the argmax itself as it stores the
         logits (kq_gemv_q8k_argmax).  The index is written to pinned host memory and read after the stream: no
-        copy back (151936x4096 Q6_K / 248320x4096 Q4_K head call 119 / 129 -> 111 / 122 us, with the
-        cheaper Python of ops)."""
+        copy back (151936x4096 Q6_K / 248320x4096 Q4_K against a device index and its copy: 113.9 / 124.6 ->
+        113.4 / 123.3 us a call, the first one on new weights 180 / 200 -> 157 / 176 us)."""
         w, R, C, ty = self.w[name]
         if y is None:
             if self.logits.numel() < R:
@@ -324,7 +324,7 @@ class Engine:
             return self._rows_f32(mats, X, outs)
         xq = self._quantize(X, C)
         # three matrices a call, one launch per weight type or one for both (the 1024-row k and v alone leave most CUs
-        # idle): 4 tokens through the 9B layer 52.8 -> 46.1 us, 16 tokens 79.5 -> 63.5 us
+        # idle): 4 / 16 tokens through the 9B layer 52.8 / 79.5 -> 43.9 / 59.9 us
         for i in range(0, len(mats), 3):
             ops.gemv_q8k_multi(mats[i:i + 3], xq, N, outs[i:i + 3])
         return 1

@@ -248,7 +248,7 @@ def gemv_q8k_x(mats, x, ys, xq=None):
 
 def gemv_q8k_multi(mats, xq, N, ys):
     """Up to 3 matrices [(w, R, C, type)] sharing one Q8_K input, one launch per type, or one for
-    both types at one token and C <= 4096 when one type has a single matrix (kq_gemv_q8k_multi).
+    both types at C <= 4096 under the conditions of kq_gemv_q8k_multi.
     ys[i] is [N][ld_i] or [R_i]."""
     n = len(mats)
     if not 1 <= n <= 3 or len(ys) != n:
@@ -362,7 +362,7 @@ def f32_multi_workspace(Rs, C_, M):
 
 class HostIndex:
     """An int32 in pinned host memory that the argmax kernels write (``out`` of argmax / gemv_q8k_argmax) and the host
-    reads after its stream: no copy back from the device (head call of 151936x4096 Q6_K: see Engine.head)."""
+    reads after its stream: no copy back from the device (figures: Engine.head)."""
 
     def __init__(self):
         self._t = torch.empty(1, dtype=torch.int32, pin_memory=True)
